@@ -205,6 +205,8 @@ def main():
     achieved = bytes_per_launch / dur_per_launch / 1e9
     kernel_name = {0: "k_trace_closest", 2: "k_trace_persistent",
                    3: "k_trace_persistent_lds"}[rm.get_tuning(rm.TUNE_TRACE_VARIANT)]
+    if kernel_name == "k_trace_persistent_lds" and rm.get_tuning(rm.TUNE_TRIS_PER_STEP) == 0:
+        kernel_name = "k_trace_wide"  # whole leaves: the four-wide walk
     # HBM bytes per launch from the committed PMC passes of this kernel (the
     # launch parameters they were taken at are reported beside them)
     traffic, traffic_launch = None, None

@@ -471,19 +471,22 @@ int32_t rm_generate_rays(int32_t kind, uint32_t seed, int64_t n, const rm_render
  * Process-wide; set them before launching work. */
 enum rm_tune_key {
     RM_TUNE_TRACE_VARIANT = 0,          /* 0 stack walk (one ray per lane), 2 persistent step walk,
-                                           3 persistent step walk with the first stack entries in LDS
-                                           (default; in a render launch: every walk of its kernels);
-                                           1 and 4 (a one-ray step walk and two walks per lane) are
+                                           3 persistent walk with its stack in LDS (default; in a render
+                                           launch: every walk of its kernels): with RM_TUNE_TRIS_PER_STEP
+                                           0 the walk of a four-wide tree (scenes of at most 48 triangles
+                                           are tested without a tree), else the step walk of the binary
+                                           tree; 1 and 4 (a one-ray step walk and two walks per lane) are
                                            retired and rejected */
     RM_TUNE_PERSISTENT_BLOCKS_PER_CU = 1, /* resident 256-lane blocks per CU for variants 2, 3 (default 8) */
-    RM_TUNE_FETCH_MIN = 2,              /* idle lanes before a wave claims new rays (default 48) */
+    RM_TUNE_FETCH_MIN = 2,              /* idle lanes before a wave claims new rays (default 16) */
     RM_TUNE_RAY_SORT = 3,               /* ray reordering for trace calls: 0 never, 1 when consecutive
                                            origins are far apart, 2 always, 3 as 1 with a radix sort
                                            of the bins (rocPRIM) instead of the counting sort, 4 as 3
                                            with the library's own radix sort, whose kernels do no work
                                            on a batch left unsorted, 5 as 4 with a closest-hit batch of
                                            shared origins (a camera's) sorted by direction into small
-                                           tiles instead (default) */
+                                           tiles instead (default); the four-wide walk reorders in modes
+                                           4 and 5 only large incoherent batches of large scenes */
     RM_TUNE_RENDER_BLOCKS_PER_CU = 4,   /* blocks per CU of the persistent bounce kernel (default 4) */
     RM_TUNE_ADJOINT_SPLIT = 5,          /* lanes per pixel of the adjoint, each replaying a share of
                                            the pixel's samples (default 4) */

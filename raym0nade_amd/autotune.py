@@ -5,7 +5,7 @@ the summation order of accumulator sets), so the tuner only times candidates
 on the caller's own workload and keeps the fastest:
 
   tune_trace   traversal variant (stack walk / persistent step walk with
-               the stack in scratch or partly in LDS), resident blocks per CU, the idle-lane threshold at which
+               the stack in scratch or partly in LDS, or the four-wide walk), resident blocks per CU, the idle-lane threshold at which
                a persistent wave fetches new rays, ray reordering, LDS stack
                entries, triangles per step and walk phases, on the caller's
                ray batches;
@@ -50,6 +50,8 @@ def tune_trace(scene, batches, reps=3, candidates=None, log=None) -> dict:
         candidates += [(3, b, f, s, e, p, ph) for b, f, e, p, s, ph in
                        itertools.product((8,), (32, 48), (8, 10), (0, 2, 4), (1, 3, 4, 5), (24, 32, 40))]
 
+        candidates += [(3, b, f, s, 10, 0, ph) for b, f, s, ph in itertools.product((6, 8), (8, 16), (0, 5), (24, 32, 40))]
+
     def run():
         for r in batches:
             scene.trace_closest(r)
@@ -73,7 +75,7 @@ def tune_trace(scene, batches, reps=3, candidates=None, log=None) -> dict:
 
 def tune_render(jobs, spp_scale=0.125, blocks=(4, 8, 16), waves=(1, 3), paths_per_round=(0, 2, 4, 8),
                 walks=((3, 10, 2, 0), (3, 10, 0, 0), (3, 10, 1, 0), (3, 10, 4, 0), (3, 8, 2, 0), (3, 6, 2, 0),
-                       (2, 32, 2, 0), (3, 10, 0, 32), (3, 10, 0, 40), (3, 10, 1, 32), (3, 10, 2, 32)),
+                       (2, 32, 2, 0), (3, 10, 0, 32), (3, 10, 0, 40), (3, 10, 1, 32), (3, 10, 2, 32), (3, 10, 0, 24)),
                 full_paths=(4, 8), log=None) -> dict:
     """jobs: list of (Scene, RmRenderArgs, Frame, post_options) as for
     render_batch.  Times the batch (hipGraph launch) with every job's spp

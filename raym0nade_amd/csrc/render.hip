@@ -1028,6 +1028,27 @@ __device__ __forceinline__ void flush_walk_counts(const Job *__restrict__ J, int
     c = TraceCounts{};
 }
 
+// The wide walk of a queue.  ONE: every lane's scene is job 0's.
+template <class Src>
+struct OneScene : Src {
+    SceneView S;
+    __device__ __forceinline__ const SceneView &scene() const { return S; }
+};
+template <bool ANY, bool ONE, class Src>
+__device__ __forceinline__ void wide_render_loop(const Src &src, const Job *__restrict__ J, uint32_t *work, int fetch_min,
+                                                 int phases) {
+    const uint32_t waves = gridDim.x * (RB / 64u);
+    uint32_t per = wide_per_wave(src.count, waves);
+    if constexpr (ONE) {
+        OneScene<Src> s{src, J[0].S};
+        if (s.S.flat && per < 64u) per = 64u;
+        wide_loop<ANY>(s, work, per, T_EPS, fetch_min, phases);
+    } else {
+        Src s = src;
+        wide_loop<ANY>(s, work, per, T_EPS, fetch_min, phases);
+    }
+}
+
 template <bool LDS, int TPS, bool COUNT = false>
 __global__ __launch_bounds__(RB) void k_extend(const Job *__restrict__ J, PathQ Q, const uint32_t *count_in,
                                                uint32_t *work, uint2 *__restrict__ hit, int fetch_min,
@@ -1082,6 +1103,34 @@ __global__ __launch_bounds__(RB) void k_extend(const Job *__restrict__ J, PathQ 
         }
     }
     if (COUNT) flush_walk_counts(J, job, c);
+}
+
+// k_extend with the wide walk (wide.h).
+struct ExtendSrc {
+    const Job *J;
+    const PathQ &Q;
+    uint2 *hit;
+    uint32_t count;
+    int job;
+    __device__ __forceinline__ uint32_t n() const { return count; }
+    __device__ __forceinline__ const SceneView &scene() const { return J[job].S; }
+    __device__ __forceinline__ void load(uint32_t &i, V3 &o, V3 &d, float &tmax, float &aim) {
+        const float4 a = Q.f[0][i], b = Q.f[1][i];
+        job = (int)(bu(Q.f[7][i].w) >> 8);
+        o = V3{a.x, a.y, a.z};
+        d = V3{b.x, b.y, b.z};
+        tmax = INFINITY;
+        aim = -INFINITY;
+    }
+    __device__ __forceinline__ void store(uint32_t i, float t, int32_t best, float) const {
+        hit[i] = make_uint2(bu(t), (uint32_t)best);
+    }
+};
+// ONE: a launch of one job, whose scene is the same for every lane.
+template <bool ONE>
+__global__ __launch_bounds__(RB, 8) void k_extend_wide(const Job *__restrict__ J, PathQ Q, const uint32_t *count_in,
+                                                       uint32_t *work, uint2 *__restrict__ hit, int fetch_min, int phases) {
+    wide_render_loop<false, ONE, ExtendSrc>(ExtendSrc{J, Q, hit, *count_in, 0}, J, work, fetch_min, phases);
 }
 
 // MINW: minimum resident waves per SIMD the register allocation must allow
@@ -1489,6 +1538,30 @@ __global__ __launch_bounds__(RB) void k_shadow(const Job *__restrict__ J, Shadow
     if (COUNT) flush_walk_counts(J, (int)job, c);
 }
 
+// k_shadow with the wide walk (wide.h).
+struct ShadowSrc {
+    const Job *J;
+    const ShadowQ &Q;
+    uint32_t count;
+    int job;
+    __device__ __forceinline__ uint32_t n() const { return count; }
+    __device__ __forceinline__ const SceneView &scene() const { return J[job].S; }
+    __device__ __forceinline__ void load(uint32_t &i, V3 &o, V3 &d, float &tmax, float &aim) {
+        const float4 a = Q.o[i], b = Q.d[i];
+        job = (int)bu(b.w);
+        o = V3{a.x, a.y, a.z};
+        d = V3{b.x, b.y, b.z};
+        aim = a.w;
+        tmax = aim + T_EPS;
+    }
+    __device__ __forceinline__ void store(uint32_t i, float t, int32_t, float aim) const { Q.vis[i] = t < aim ? 0 : 1; }
+};
+template <bool ONE>
+__global__ __launch_bounds__(RB, 8) void k_shadow_wide(const Job *__restrict__ J, ShadowQ SQ, const uint32_t *count,
+                                                       uint32_t *work, int fetch_min, int phases) {
+    wide_render_loop<true, ONE, ShadowSrc>(ShadowSrc{J, SQ, *count, 0}, J, work, fetch_min, phases);
+}
+
 template <int MINW>
 __global__ __launch_bounds__(RB, MINW) void k_nee_add(const Job *__restrict__ J, PixBufs P, AccBufs AB, NeeQ NQ,
                                                 const uint32_t *count, uint32_t *work, ShadowQ SQ) {
@@ -1799,11 +1872,17 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
     // Trace variant 3 keeps the first pending entries of every walk in LDS:
     // each kernel of the launch that traverses gets nl entries per lane (at
     // most the deepest tree's depth), and the job table's views say so.
-    const bool lds_walk = tuning().trace_variant == 3;
+    // The wide walk keeps every pending group there; counting renders walk in
+    // the reference's order.
+    const bool counting = tuning().render_count != 0;
+    // So do launches with a scene that has no wide tree, but for flat ones.
+    bool wide = wide_chosen(tuning()) && !counting;
+    for (int i = 0; i < nj; ++i) wide = wide && (J[i].S.wide || J[i].S.flat);
+    const bool lds_walk = tuning().trace_variant == 3 && !wide;
     int max_depth = 1;
     for (int i = 0; i < nj; ++i) max_depth = std::max(max_depth, (int)J[i].S.depth);
-    const int nl = lds_walk ? std::min(max_depth, tuning().lds_stack_entries) : 0;
-    const size_t walk_lds = (size_t)nl * RB * 8;
+    const int nl = lds_walk || wide ? std::min(max_depth, tuning().lds_stack_entries) : 0;
+    const size_t walk_lds = (size_t)nl * RB * 8, wide_lds = wide_lds_bytes(max_depth);
     // LdsStack's launch contract: every kernel below that walks is launched
     // with blocks of RB lanes and walk_lds bytes of dynamic LDS
     if (RB != WALK_BLOCK || walk_lds < (size_t)nl * WALK_BLOCK * 8 || nl > MAX_STACK)
@@ -1824,9 +1903,9 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
     // triangles per walk step: any of 0, 1, 2, 4 for the extension kernel;
     // the shading kernels' walks take a whole leaf (0) or two triangles
     const int tps = tuning().tris_per_step;
-    hipLaunchKernelGGL(maps ? (tps ? k_primary<2, true> : k_primary<0, true>)
-                            : (tps ? k_primary<2, false> : k_primary<0, false>),
-                       dim3(gp), dim3(RB), walk_lds, st, (const Job *)dJ, nj, total_px, P);
+    hipLaunchKernelGGL(maps ? (wide ? k_primary<WALK_WIDE, true> : tps ? k_primary<2, true> : k_primary<0, true>)
+                            : (wide ? k_primary<WALK_WIDE, false> : tps ? k_primary<2, false> : k_primary<0, false>),
+                       dim3(gp), dim3(RB), wide ? wide_lds : walk_lds, st, (const Job *)dJ, nj, total_px, P);
     hipLaunchKernelGGL(k_block_sums, dim3((unsigned)nblk), dim3(SB), 0, st, P.M, total_px, bsum);
     RM_HIP(hipGetLastError());
     std::vector<int64_t> hs(nblk);
@@ -1854,7 +1933,6 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
     // single-kernel passes when no job is that deep
     constexpr int SPLIT_DEPTH = 12;
     // counting renders send every shadow ray through the counting k_shadow
-    const bool counting = tuning().render_count != 0;
     const int split_mode = counting ? 1 : tuning().nee_split;
     const bool split = (split_mode == 1 || (split_mode == 2 && max_depth >= SPLIT_DEPTH)) &&
                        total * NEE_MAX <= 0xffffffffLL && total_px * dC <= 0xffffffffLL;
@@ -1925,11 +2003,19 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
                                  : tps == 4 ? k_shadow<true, 4> : k_shadow<true, 0>)
                               : (tps == 1 ? k_shadow<false, 1> : tps == 2 ? k_shadow<false, 2>
                                  : tps == 4 ? k_shadow<false, 4> : k_shadow<false, 0>));
+    auto launch_shadow = [&](const uint32_t *n, uint32_t *claim) {
+        if (wide)
+            hipLaunchKernelGGL(nj == 1 ? k_shadow_wide<true> : k_shadow_wide<false>, dim3(gpers), dim3(RB), wide_lds, st,
+                               (const Job *)dJ, SQ, n, claim, fetch_min, phases);
+        else
+            hipLaunchKernelGGL(shadow, dim3(gpers), dim3(RB), walk_lds, st, (const Job *)dJ, SQ, n, claim, fetch_min, nl,
+                               phases);
+    };
     if (split) {
         uint32_t *claims = counts + 3 * NCOUNT + 8;  // and [9]: queued rays; both zeroed for each chunk
-        auto direct_gen = mw == 4 ? (tps ? k_direct_gen<4, 2> : k_direct_gen<4, 0>)
-                          : mw == 3 ? (tps ? k_direct_gen<3, 2> : k_direct_gen<3, 0>)
-                                    : (tps ? k_direct_gen<1, 2> : k_direct_gen<1, 0>);
+        auto direct_gen = mw == 4 ? (wide ? k_direct_gen<4, WALK_FLAT> : tps ? k_direct_gen<4, 2> : k_direct_gen<4, 0>)
+                          : mw == 3 ? (wide ? k_direct_gen<3, WALK_FLAT> : tps ? k_direct_gen<3, 2> : k_direct_gen<3, 0>)
+                                    : (wide ? k_direct_gen<1, WALK_FLAT> : tps ? k_direct_gen<1, 2> : k_direct_gen<1, 0>);
         // samples [t0, t0 + C) of the pixels [0, npx) whose jobs have more than
         // t0 samples (jobs are in order of falling sample counts)
         for (int t0 = 0; t0 < max_direct;) {
@@ -1942,16 +2028,15 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
             hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(128), 0, st, claims, 2);
             hipLaunchKernelGGL(direct_gen, dim3((unsigned)((n + RB - 1) / RB)), dim3(RB), walk_lds, st,
                                (const Job *)dJ, nj, npx, P, C, t0, SQ, queue_depth, claims + 1);
-            hipLaunchKernelGGL(shadow, dim3(gpers), dim3(RB), walk_lds, st, (const Job *)dJ, SQ,
-                               (const uint32_t *)(claims + 1), claims, fetch_min, nl, phases);
+            launch_shadow((const uint32_t *)(claims + 1), claims);
             hipLaunchKernelGGL(k_direct_add, dim3((unsigned)((npx + RB - 1) / RB)), dim3(RB), 0, st, (const Job *)dJ, nj,
                                npx, P, C, t0, SQ);
             t0 += C;
         }
         hipLaunchKernelGGL(k_direct_final, dim3(gp), dim3(RB), 0, st, (const Job *)dJ, nj, total_px);
     } else {
-        auto direct = mw == 4 ? (tps ? k_direct<4, 2> : k_direct<4, 0>)
-                      : mw == 3 ? (tps ? k_direct<3, 2> : k_direct<3, 0>) : (tps ? k_direct<1, 2> : k_direct<1, 0>);
+        auto direct = mw == 4 ? (wide ? k_direct<4, WALK_FLAT> : tps ? k_direct<4, 2> : k_direct<4, 0>)
+                      : mw == 3 ? (wide ? k_direct<3, WALK_FLAT> : tps ? k_direct<3, 2> : k_direct<3, 0>) : (wide ? k_direct<1, WALK_FLAT> : tps ? k_direct<1, 2> : k_direct<1, 0>);
         hipLaunchKernelGGL(direct, dim3(gp), dim3(RB), walk_lds, st, (const Job *)dJ, nj, total_px, P);
     }
     const uint32_t nsets = (uint32_t)total;
@@ -1962,10 +2047,10 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
         const unsigned ge = gpers;
         auto bounce = maps ? (mw == 4 ? k_bounce<4, true> : mw == 3 ? k_bounce<3, true> : k_bounce<1, true>)
                            : (mw == 4 ? k_bounce<4, false> : mw == 3 ? k_bounce<3, false> : k_bounce<1, false>);
-        auto nee = mw == 4 ? (tps ? k_nee<4, 2> : k_nee<4, 0>)
-                   : mw == 3 ? (tps ? k_nee<3, 2> : k_nee<3, 0>) : (tps ? k_nee<1, 2> : k_nee<1, 0>);
-        auto nee_gen = mw == 4 ? (tps ? k_nee_gen<4, 2> : k_nee_gen<4, 0>)
-                       : mw == 3 ? (tps ? k_nee_gen<3, 2> : k_nee_gen<3, 0>) : (tps ? k_nee_gen<1, 2> : k_nee_gen<1, 0>);
+        auto nee = mw == 4 ? (wide ? k_nee<4, WALK_FLAT> : tps ? k_nee<4, 2> : k_nee<4, 0>)
+                   : mw == 3 ? (wide ? k_nee<3, WALK_FLAT> : tps ? k_nee<3, 2> : k_nee<3, 0>) : (wide ? k_nee<1, WALK_FLAT> : tps ? k_nee<1, 2> : k_nee<1, 0>);
+        auto nee_gen = mw == 4 ? (wide ? k_nee_gen<4, WALK_FLAT> : tps ? k_nee_gen<4, 2> : k_nee_gen<4, 0>)
+                       : mw == 3 ? (wide ? k_nee_gen<3, WALK_FLAT> : tps ? k_nee_gen<3, 2> : k_nee_gen<3, 0>) : (wide ? k_nee_gen<1, WALK_FLAT> : tps ? k_nee_gen<1, 2> : k_nee_gen<1, 0>);
         auto nee_add = mw == 4 ? k_nee_add<4> : mw == 3 ? k_nee_add<3> : k_nee_add<1>;
         auto extend_lds = counting ? (tps == 1 ? k_extend<true, 1, true> : tps == 2 ? k_extend<true, 2, true>
                                       : tps == 4 ? k_extend<true, 4, true> : k_extend<true, 0, true>)
@@ -1980,7 +2065,11 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
             hipLaunchKernelGGL(k_spawn, dim3(gs), dim3(RB), 0, st, (const Job *)dJ, nj, P, j, nsets, Q[0], counts);
             for (int d = 1; d <= D; ++d) {
                 const uint32_t *n_in = counts + d - 1;
-                if (lds_walk)
+                if (wide)
+                    hipLaunchKernelGGL(nj == 1 ? k_extend_wide<true> : k_extend_wide<false>, dim3(ge), dim3(RB), wide_lds,
+                                       st, (const Job *)dJ, Q[(d - 1) & 1], n_in, counts + 2 * NCOUNT + d, hits, fetch_min,
+                                       phases);
+                else if (lds_walk)
                     hipLaunchKernelGGL(extend_lds, dim3(ge), dim3(RB), walk_lds, st, (const Job *)dJ,
                                        Q[(d - 1) & 1], n_in, counts + 2 * NCOUNT + d, hits, fetch_min, nl, phases);
                 else
@@ -1994,9 +2083,7 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
             if (split) {
                 hipLaunchKernelGGL(nee_gen, dim3(gb), dim3(RB), walk_lds, st, (const Job *)dJ, nj, NQ, n_nee,
                                    counts + 3 * NCOUNT + 1, SQ, queue_depth, counts + 3 * NCOUNT + 4);
-                hipLaunchKernelGGL(shadow, dim3(ge), dim3(RB), walk_lds, st, (const Job *)dJ, SQ,
-                                   (const uint32_t *)(counts + 3 * NCOUNT + 4), counts + 3 * NCOUNT + 2, fetch_min, nl,
-                                   phases);
+                launch_shadow((const uint32_t *)(counts + 3 * NCOUNT + 4), counts + 3 * NCOUNT + 2);
                 hipLaunchKernelGGL(nee_add, dim3(gb), dim3(RB), 0, st, (const Job *)dJ, P, AB, NQ, n_nee,
                                    counts + 3 * NCOUNT + 3, SQ);
             } else {

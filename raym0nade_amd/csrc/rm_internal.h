@@ -129,9 +129,10 @@ int32_t build_host_scene(const rm_scene_desc *d, HostScene &hs);
 
 // Launch parameters chosen by the autotuner (rm_set_tuning).
 struct Tuning {
-    int trace_variant = 3;        // 0 stack walk, 2 persistent step walk, 3 same with LDS stacks
+    int trace_variant = 3;        // 0 stack walk, 2 persistent step walk, 3 same with LDS stacks, or with
+                                  // tris_per_step 0 the four-wide walk (wide.h)
     int persistent_blocks_per_cu = 8;
-    int fetch_min = 48;           // idle lanes before a wave claims new rays
+    int fetch_min = 16;           // idle lanes before a wave claims new rays
     int ray_sort = 5;             // 0 never, 1 when consecutive origins are far apart, 2 always,
                                   // 3 as 1 with a radix sort (rocPRIM) instead of the counting sort,
                                   // 4 as 3 with the library's own radix sort (skipped on the device
@@ -142,13 +143,15 @@ struct Tuning {
     int kernel_timing = 0;        // record HIP events around the trace kernels (rm_last_trace_ms)
     int render_min_waves = 1;     // 1 or 4: register cap of the shading and NEE kernels
     int lds_stack_entries = 10;   // trace variant 3: walk-stack entries per lane kept in LDS (160 KiB at 8 blocks/CU)
-    int tris_per_step = 0;        // trace variant 3: triangles tested per step (0: a whole leaf)
+    int tris_per_step = 0;        // trace variant 3: triangles tested per step (0: the four-wide walk)
     int nee_split = 2;            // render: shadow rays of light samples in their own passes (2: deep trees)
     int render_count = 0;         // render: count the extension and shadow walks (RM_STAT_WALK_*)
     int trace_util = 0;           // trace variant 3: count lane utilisation (rm_last_trace_util)
     int walk_phases = 32;         // persistent walks: one kind of step per iteration (RM_TUNE_WALK_PHASES)
 };
 Tuning &tuning();
+// Whether walks are the four-wide one by default (variant 3, whole leaves).
+inline bool wide_chosen(const Tuning &t) { return t.trace_variant == 3 && t.tris_per_step == 0; }
 int device_cu_count();
 
 }  // namespace rm
@@ -156,7 +159,7 @@ int device_cu_count();
 struct rm_scene {
     rm::HostScene host;  // perm + sizes kept; big arrays released after upload
     rm::SceneView view{};
-    rm::DevBuf nodes, tris, shade, mats, texs, texels, bytes, lights, light_faces, light_cdf, sky, sky_cdf, sky_guide;
+    rm::DevBuf wide, nodes, tris, shade, mats, texs, texels, bytes, lights, light_faces, light_cdf, sky, sky_cdf, sky_guide;
     rm_scene_info info{};
     uint64_t version = 0;  // bumped by rm_scene_update
 };
@@ -165,4 +168,6 @@ namespace rm {
 // Box-filtered mip levels 1.. of texture `t` from its level 0 in the device
 // texel pool, the same arithmetic as the host build (stream-ordered).
 int32_t launch_mip_build(const rm_scene *s, int t, hipStream_t st);
+// The four-wide tree of an uploaded scene (wide.h); waits for it.
+int32_t build_wide(rm_scene *s);
 }  // namespace rm

@@ -33,7 +33,8 @@ static_assert(sizeof(PairNode) == 64, "PairNode is 64 B");
 //                        stand-in for |a| / length(edge1) < 1e-4
 //                        (src/geometry.cpp:70); see flatten code.
 //   e1 = v1 - v0, orig   orig: original triangle id as int bits
-//   e2 = v2 - v0, 0
+//   e2 = v2 - v0, leaf   leaf: number of the triangle's leaf in the implicit
+//                        heap, as int bits (filled with the wide tree)
 // Edges are the same fp32 differences the reference computes per test
 // (src/geometry.cpp:65-66), so every test result is bit-identical.
 struct alignas(16) TriRec {
@@ -42,6 +43,18 @@ struct alignas(16) TriRec {
     float e2[4];
 };
 static_assert(sizeof(TriRec) == 48, "TriRec is 48 B");
+
+// Node of the four-wide tree (wide.h), 64 B.  Per axis the children's lower
+// planes (four fp16, two words) then their upper planes, as offsets from the
+// node's origin in scaled coordinates; an empty child has an infinite lower
+// and a zero upper plane.  m[0] = origin x | y << 16, m[1] = origin z | E << 16,
+// m[2] = D (fp16), m[3] = reference of child 0 (child k: + k).  E and D are 0
+// except over the runs of a leaf: the largest |e2| of its triangles and the
+// diagonal of their bounds, scaled, fp16 rounded up.
+struct alignas(64) WideNode {
+    uint32_t x[4], y[4], z[4], m[4];
+};
+static_assert(sizeof(WideNode) == 64, "WideNode is one cache line");
 
 // Walk-stack capacity: pending entries <= tree depth - 1 (2^27 faces -> 25).
 constexpr int MAX_STACK = 32;
@@ -133,6 +146,11 @@ struct SceneView {
     // 1 when a material is an alpha cut-out: walks then apply TransparentTest.
     int32_t cutout;
     const uint8_t *bytes;         // 8-bit texels of every 8-bit texture, all mip levels
+    // the four-wide tree (wide.h) over the scene, nullptr when it has none;
+    // its coordinates are (x - wide_lo) * wide_scale, a power of two
+    const WideNode *wide;
+    int32_t flat;                 // the number of triangles when rays test them all (wide.h), else 0
+    float wide_lo[3], wide_scale, wide_rscale;
 };
 
 }  // namespace rm

@@ -638,6 +638,7 @@ extern "C" int32_t rm_scene_create(const rm_scene_desc *desc, rm_scene **out) {
     v.sky_w = h.sky_w;
     v.sky_h = h.sky_h;
     v.n_mats = (int32_t)h.mats.size();
+    if ((st = build_wide(s))) { delete s; return st; }
     rm_scene_info &I = s->info;
     I.n_tris = h.n;
     I.n_nodes = h.n_nodes;
@@ -645,7 +646,7 @@ extern "C" int32_t rm_scene_create(const rm_scene_desc *desc, rm_scene **out) {
     I.n_light_objects = (int32_t)h.lights.size();
     I.n_light_faces = (int32_t)h.light_faces.size();
     I.has_sky = h.sky.empty() ? 0 : 1;
-    I.device_bytes = (int64_t)(s->nodes.bytes + s->tris.bytes + s->shade.bytes + s->mats.bytes + s->texs.bytes +
+    I.device_bytes = (int64_t)(s->wide.bytes + s->nodes.bytes + s->tris.bytes + s->shade.bytes + s->mats.bytes + s->texs.bytes +
                                s->texels.bytes + s->bytes.bytes + s->lights.bytes + s->light_faces.bytes +
                                s->light_cdf.bytes +
                                s->sky.bytes + s->sky_cdf.bytes + s->sky_guide.bytes);

@@ -8,7 +8,7 @@
 #include "rm_layout.h"
 #include "rm_vec.h"
 #include "tex8.h"
-#include "traverse.h"
+#include "wide.h"
 
 namespace rm {
 
@@ -811,7 +811,7 @@ __device__ __noinline__ int32_t model_hit_rest(const SceneView &S, V3 o, V3 d, f
         if (T == 7) break;
         const float tmin = t + T_EPS;
         t = tmax0;
-        slot = trace_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
+        slot = scene_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
     }
     t = tmax0;
     return -1;
@@ -825,7 +825,7 @@ __device__ __forceinline__ int32_t model_closest(const SceneView &S, V3 o, V3 d,
     float tmin = T_EPS;
     for (int T = 0;; ++T) {
         t = INFINITY;
-        const int32_t slot = trace_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
+        const int32_t slot = scene_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
         if (!S.cutout || slot < 0 || !transparent_at(S, o, d, t, slot)) return slot;
         if (T == 7) break;
         tmin = t + T_EPS;
@@ -845,7 +845,7 @@ __device__ __forceinline__ bool model_clear(const SceneView &S, V3 o, V3 d, cons
     const float stop = S.cutout ? -INFINITY : aim;
     for (int T = 0; T < 8; ++T) {
         float tmax = aim + T_EPS;
-        const int32_t slot = trace_walk<true, LDSW, TPS>(S, r, tmin, tmax, stop);
+        const int32_t slot = scene_walk<true, LDSW, TPS>(S, r, tmin, tmax, stop);
         if (!(tmax < aim)) return true;
         if (!S.cutout || !transparent_at(S, o, d, tmax, slot)) return false;
         tmin = tmax + T_EPS;
@@ -863,7 +863,7 @@ __device__ __noinline__ bool model_blocked(const SceneView &S, V3 o, V3 d, float
     const RayPre r = ray_pre(o, d);
     for (int T = 0; T < 8; ++T) {
         float t = aim + T_EPS;
-        const int32_t slot = trace_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
+        const int32_t slot = scene_walk<false, LDSW, TPS>(S, r, tmin, t, -INFINITY);
         if (t >= aim) return false;
         if (!transparent_at(S, o, d, t, slot)) return true;
         tmin = t + T_EPS;

@@ -194,6 +194,48 @@ __global__ __launch_bounds__(TRACE_BLOCK) void k_trace_persistent(SceneView S, c
     }
 }
 
+// The wide walk (wide.h) of a ray batch.
+template <bool ANY>
+struct TraceSrc {
+    const SceneView &S;
+    const float *rays;
+    const float *aim_arr;
+    const uint32_t *order;
+    float *t_out;
+    int32_t *id_out;
+    uint8_t *occ;
+    uint32_t count;
+    float t0;
+    __device__ __forceinline__ uint32_t n() const { return count; }
+    __device__ __forceinline__ const SceneView &scene() const { return S; }
+    __device__ __forceinline__ void load(uint32_t &i, V3 &o, V3 &d, float &tmax, float &aim) const {
+        if (order) i = order[i];
+        load_ray(rays, i, o, d);
+        aim = ANY ? (aim_arr ? aim_arr[i] : t0) : -INFINITY;
+        tmax = ANY ? aim + T_EPS : t0;
+    }
+    __device__ __forceinline__ void store(uint32_t i, float t, int32_t best, float aim) const {
+        if (ANY) {
+            occ[i] = t < aim ? 1 : 0;
+        } else {
+            t_out[i] = t;
+            id_out[i] = out_id(S, best);
+        }
+    }
+};
+
+template <bool ANY>
+__global__ __launch_bounds__(TRACE_BLOCK, 8) void k_trace_wide(SceneView S, const float *__restrict__ rays, uint32_t n,
+                                                               float tmin, float t0, const float *__restrict__ aim_arr,
+                                                               float *__restrict__ t_out, int32_t *__restrict__ id_out,
+                                                               uint8_t *__restrict__ occ, unsigned long long *work,
+                                                               uint32_t per, int fetch_min,
+                                                               const uint32_t *__restrict__ order,
+                                                               const int *__restrict__ use_order, int phases) {
+    TraceSrc<ANY> src{S, rays, aim_arr, order && *use_order ? order : nullptr, t_out, id_out, occ, n, t0};
+    wide_loop<ANY>(src, work, per, tmin, fetch_min, phases);
+}
+
 __global__ void k_zero_u64(unsigned long long *p) { *p = 0ull; }
 
 // ---------------------------------------------------------------- reordering
@@ -704,6 +746,15 @@ struct FixedWorkspace {
     size_t bytes;
 };
 
+// Sort modes 4 and 5 reorder a batch for the wide walk from this many rays
+// (any hits: twice as many) and triangles on; coherent batches never.  Sorted
+// / unsorted, closest hits of uniform rays: 1M triangles, 300k rays 603 / 514
+// us, 1M 1025 / 1234, 2M 1592 / 2172, 8M 4770 / 7840; 200k triangles, 1M 750 /
+// 740, 2M 1029 / 1178; 5k triangles (all in one L2), 2M 672 / 574.  Any hits
+// among 1M triangles: 1M 707 / 700, 2M 1021 / 1107.  A camera's 8M rays sorted
+// by direction: 2788 / 2544.
+constexpr int64_t WIDE_SORT_RAYS = 1000000, WIDE_SORT_TRIS = 100000;
+
 template <bool ANY>
 static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, float tmin, float t0, const float *aim_dev,
                             float *t_out, int32_t *id_out, uint8_t *occ, hipStream_t st,
@@ -718,7 +769,11 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
     int *flag = nullptr;
     char *ws = nullptr;
     std::unique_lock<std::mutex> ws_lock;
-    if ((T.ray_sort == 4 || T.ray_sort == 5) && n >= 4096) {
+    // The wide walk is sorted less: only large incoherent batches gain.
+    const bool wide = wide_chosen(T) && (s->view.wide || s->view.flat) && !(T.trace_util && !fixed) &&
+                      n < (int64_t)0xf0000000;
+    const int64_t sort_min = !wide ? 4096 : s->view.n_tris < WIDE_SORT_TRIS ? INT64_MAX : ANY ? 2 * WIDE_SORT_RAYS : WIDE_SORT_RAYS;
+    if ((T.ray_sort == 4 || T.ray_sort == 5) && n >= sort_min) {
         // the library's radix sort: keys, keys2, values, values2, flag, tile histograms, chunk totals
         const size_t plane = ((size_t)n * 4 + 255) & ~(size_t)255;
         const uint32_t nt = (uint32_t)((n + RS_TILE - 1) / RS_TILE);
@@ -750,7 +805,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         const unsigned gn = (unsigned)((n + 255) / 256);
         // mode 5: flag, then the direction range of a coherent batch, in the flag's 256-byte slot;
         // closest-hit calls only (any-hit walks stop at the first hit and do not pay for the sort)
-        float *box = (T.ray_sort == 5 && !ANY) ? reinterpret_cast<float *>(flag + 1) : nullptr;
+        float *box = (T.ray_sort == 5 && !ANY && !wide) ? reinterpret_cast<float *>(flag + 1) : nullptr;
         hipLaunchKernelGGL(k_coherence, dim3(1), dim3(256), 0, st, s->view, rays, n, 0.02f, flag, box);
         hipLaunchKernelGGL(k_bin_keys, dim3(gn), dim3(256), 0, st, s->view, rays, n, (const int *)flag, keys, vals, 1,
                            (const float *)box);
@@ -798,7 +853,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         hipLaunchKernelGGL(k_bin_keys, dim3(gn), dim3(256), 0, st, s->view, rays, n, (const int *)flag, keys, vals);
         RM_HIP(rocprim::radix_sort_pairs(tmp, tmp_bytes, (const uint32_t *)keys, keys2, (const uint32_t *)vals, order,
                                          (size_t)n, 0u, (unsigned)(3 * CELL_BITS + 3), st));
-    } else if (T.ray_sort != 0 && n >= 4096) {
+    } else if (T.ray_sort != 0 && T.ray_sort < 4 && n >= 4096) {
         size_t bytes = (size_t)n * 8 + (size_t)NBINS * 4 + 256;
         if (fixed) {
             if (fixed->bytes < bytes)
@@ -836,8 +891,17 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         unsigned pgrid = (unsigned)std::min<int64_t>(grid, (int64_t)device_cu_count() * T.persistent_blocks_per_cu);
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, next);
         const int nl = std::min(std::max(1, (int)s->view.depth), T.lds_stack_entries);
-        if (T.trace_variant == 3) {
-            const bool util = T.trace_util != 0 && !fixed;
+        const bool util = T.trace_util != 0 && !fixed;
+        if (wide) {
+            // every wave a few rays, or the whole machine
+            const uint32_t most = (uint32_t)device_cu_count() * T.persistent_blocks_per_cu * (TRACE_BLOCK / 64);
+            const uint32_t per = s->view.flat ? 64u : wide_per_wave((uint32_t)n, most);
+            const uint32_t waves = (uint32_t)std::min<int64_t>(most, (n + per - 1) / per);
+            pgrid = (waves + TRACE_BLOCK / 64 - 1) / (TRACE_BLOCK / 64);
+            hipLaunchKernelGGL(k_trace_wide<ANY>, dim3(pgrid), dim3(TRACE_BLOCK), wide_lds_bytes(s->view.depth), st,
+                               s->view, rays, (uint32_t)n, tmin, t0, aim_dev, t_out, id_out, occ, next, per,
+                               T.fetch_min, (const uint32_t *)order, (const int *)flag, T.walk_phases);
+        } else if (T.trace_variant == 3) {
             unsigned long long *ud = nullptr;
             if (util) {
                 void *p = nullptr;

@@ -73,22 +73,23 @@ __device__ __forceinline__ void box_test(const RayPre &r, float lx, float ly, fl
 }
 
 // RayTriangleIntersection (src/geometry.cpp:63-87).
-__device__ __forceinline__ float tri_test(const RayPre &r, const TriRec &T) {
+__device__ __forceinline__ float tri_test(V3 o, V3 d, const TriRec &T) {
     V3 v0{T.p[0], T.p[1], T.p[2]};
     V3 e1{T.e1[0], T.e1[1], T.e1[2]};
     V3 e2{T.e2[0], T.e2[1], T.e2[2]};
-    V3 h = cross(r.d, e2);
+    V3 h = cross(d, e2);
     float a = dot(e1, h);
     if (fabsf(a) < T.p[3]) return INFINITY;
     float f = 1.0f / a;
-    V3 s = r.o - v0;
+    V3 s = o - v0;
     float u = f * dot(s, h);
     if (u < 0.0f || u > 1.0f) return INFINITY;
     V3 q = cross(s, e1);
-    float v = f * dot(r.d, q);
+    float v = f * dot(d, q);
     if (v < 0.0f || u + v > 1.0f) return INFINITY;
     return f * dot(e2, q);
 }
+__device__ __forceinline__ float tri_test(const RayPre &r, const TriRec &T) { return tri_test(r.o, r.d, T); }
 
 __device__ __forceinline__ TriRec load_tri(const TriRec *tris, uint32_t i) {
     TriRec T;
@@ -100,6 +101,33 @@ __device__ __forceinline__ TriRec load_tri(const TriRec *tris, uint32_t i) {
     return T;
 }
 
+// 1 / a, correctly rounded.  The hardware's reciprocal (1 ulp) and one Newton
+// step with fused multiply-adds give the IEEE quotient for every significand
+// (all 2^23, both signs, compared with the division); reciprocals that are
+// not normal numbers take the division.  Three instructions and a class test
+// instead of the division's eleven.
+__device__ __forceinline__ float exact_rcp(float a) {
+    const float r = __builtin_amdgcn_rcpf(a);
+    float f = __builtin_fmaf(__builtin_fmaf(-a, r, 1.0f), r, r);
+    const float m = fabsf(a);
+    if (!(m > 0x1p-120f && m < 0x1p120f)) f = 1.0f / a;
+    return f;
+}
+
+// tri_test for walks whose lanes nearly always need the whole test: the
+// rejections are selected at the end, with the same comparisons.
+__device__ __forceinline__ float tri_test_flat(V3 o, V3 d, V3 v0, float thr, V3 e1, V3 e2) {
+    const V3 h = cross(d, e2);
+    const float a = dot(e1, h);
+    const float f = exact_rcp(a);
+    const V3 s = o - v0;
+    const float u = f * dot(s, h);
+    const V3 q = cross(s, e1);
+    const float v = f * dot(d, q);
+    const float t = f * dot(e2, q);
+    const bool out = (fabsf(a) < thr) | (u < 0.0f) | (u > 1.0f) | (v < 0.0f) | (u + v > 1.0f);
+    return out ? INFINITY : t;
+}
 struct TraceCounts {
     uint32_t interior, leaves, boxes, tris;
 };
