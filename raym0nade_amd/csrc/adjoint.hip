@@ -283,8 +283,9 @@ __device__ __forceinline__ bool nonzero(V3 v) { return v.x != 0.0f || v.y != 0.0
 // One indirect sample of an opaque first vertex (k_spawn + k_bounce of the
 // renderer, same draws in the same order).  AD = false: Lam = sum w L and
 // Cv = the image contribution (before exposure).  AD = true: the derivatives.
-template <bool AD>
-__device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3 in, float hit_t, const Diff &cam,
+// (A runtime argument: two copies of this function make the kernel 262 KB of
+// code, four times the instruction cache.)
+__device__ __forceinline__ void replay_path(const bool AD, const AdjArgs &G, const Surf &s0, V3 in, float hit_t, const Diff &cam,
                                             const ImgW &iw, int64_t p, uint32_t si, float inv, int32_t drop, V3 &Lam,
                                             V3 &Cv, V3 dl, V3 &gb, float &gr0, float *sh) {
     const SceneView &S = G.S;
@@ -302,10 +303,7 @@ __device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3
     V3 nd, bp;
     int fails = 0;
     RefTap tap0(s0.roughness);
-    if (AD)
-        sample_reflection(s0, V0, rng, nd, bp, fails, tap0);
-    else
-        sample_reflection(s0, V0, rng, nd, bp, fails);
+    sample_reflection(s0, V0, rng, nd, bp, fails, tap0);
     bp /= 1.0f;
     if (!any_finite(nd)) return;
     const V3 p0 = bp;
@@ -330,7 +328,7 @@ __device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3
     for (;;) {
         RayPre r = ray_pre(o, d);
         float t = INFINITY;
-        int32_t slot = model_closest<false, 0>(S, o, d, r, t);
+        int32_t slot = model_closest<false, WALK_FLAT>(S, o, d, r, t);
         if (slot < 0) {
             if (!exclude && S.sky) {
                 V3 L = sky_get(S, d) * v3(1.0f);
@@ -350,7 +348,7 @@ __device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3
         V3 dPdx, dPdy;
         TexFoot tf;
         tf.tex = -1;
-        hit_info<false>(S, slot, d, t, diff, dPdx, dPdy, s, AD ? &tf : nullptr);  // rm_adjoint refuses 8-bit maps
+        hit_info<false>(S, slot, d, t, diff, dPdx, dPdy, s, &tf);  // rm_adjoint refuses 8-bit maps
         V3 V = -d;
         if (rf < 1.0f * s.roughness) src = s.id;  // gmax keeps the first argument on ties
         rf = gmax(rf, 1.0f * s.roughness);
@@ -393,7 +391,7 @@ __device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3
                     LSample x;
                     DirectInfo di;
                     TraceCounts tc{};
-                    if (!direct_sample<false, false>(S, s, V, total, cnt, rng, x, tc, &di)) continue;
+                    if (!direct_sample<false, false, WALK_FLAT>(S, s, V, total, cnt, rng, x, tc, &di)) continue;
                     x.bsdf *= factor;
                     const uint32_t id = si * 8u + k;
                     ++k;
@@ -438,10 +436,7 @@ __device__ __forceinline__ void replay_path(const AdjArgs &G, const Surf &s0, V3
         calc_dDdxy(d, s.surfN, diff, nx.dDdx, nx.dDdy);
         int fl = 0;
         RefTap tp(s.roughness);
-        if (AD)
-            sample_reflection(s, V, rng, nd, bp, fl, tp);
-        else
-            sample_reflection(s, V, rng, nd, bp, fl);
+        sample_reflection(s, V, rng, nd, bp, fl, tp);
         const V3 bps = bp;
         bp /= 1.0f;
         if (doNEE) bp /= P_RR;
@@ -472,7 +467,7 @@ __device__ __forceinline__ void adjoint_pixel(const AdjArgs &G, int64_t p, int c
     camera_ray(A, x, y, Dir, cam);
     RayPre r = ray_pre(A.pos, Dir);
     float t = INFINITY;
-    int32_t slot = model_closest<false, 0>(S, A.pos, Dir, r, t);
+    int32_t slot = model_closest<false, WALK_FLAT>(S, A.pos, Dir, r, t);
     const V3 dimg = ld3(G.dimg + p * 3);
     const float ex = A.exposure;
     V3 rep = v3(0.0f);
@@ -529,7 +524,7 @@ __device__ __forceinline__ void adjoint_pixel(const AdjArgs &G, int64_t p, int c
                 LSample ls;
                 DirectInfo di;
                 TraceCounts tc{};
-                if (!direct_sample<false, false>(S, s, V, total, cnt, g, ls, tc, &di)) continue;
+                if (!direct_sample<false, false, WALK_FLAT>(S, s, V, total, cnt, g, ls, tc, &di)) continue;
                 if (length(ls.light) < T_EPS) continue;
                 if (G.replay) {
                     Acc4 dd{0, 0, 0, 0}, ds{0, 0, 0, 0};
@@ -563,7 +558,8 @@ __device__ __forceinline__ void adjoint_pixel(const AdjArgs &G, int64_t p, int c
     const int32_t drop = G.drop[p];
     const float hit_t = length(s.pos - A.pos);
     for (int si = chunk; si < n_ind; si += G.split) {
-        V3 Lam, Cv;
+        V3 Lam = v3(0.0f), Cv = v3(0.0f);
+        bool known = false;
         if (G.rec && !(drop >= 0 && (drop >> 3) == si)) {
             // the render recorded this sample's sums (its dropped outlier, if
             // any, is not excluded there, so such a sample is replayed instead)
@@ -571,12 +567,17 @@ __device__ __forceinline__ void adjoint_pixel(const AdjArgs &G, int64_t p, int c
             float4 r0 = r[0], r1 = r[1], r2 = r[2];
             Cv = Fb * V3{r0.x, r0.y, r0.z} + V3{r1.x, r1.y, r1.z};
             Lam = V3{r2.x, r2.y, r2.z};
-        } else {
-            replay_path<false>(G, s0, in, hit_t, cam, iw, p, (uint32_t)si, inv, drop, Lam, Cv, dl, gb, gr0, sh);
+            known = true;
         }
-        rep += Cv * ex;
-        if (want_grad && nonzero(Cv))
-            replay_path<true>(G, s0, in, hit_t, cam, iw, p, (uint32_t)si, inv, drop, Lam, Cv, dl, gb, gr0, sh);
+        // a sample without a record is replayed for its sums first
+#pragma nounroll
+        for (int pass = known ? 1 : 0; pass < 2; ++pass) {
+            if (pass == 1) {
+                rep += Cv * ex;
+                if (!(want_grad && nonzero(Cv))) break;
+            }
+            replay_path(pass == 1, G, s0, in, hit_t, cam, iw, p, (uint32_t)si, inv, drop, Lam, Cv, dl, gb, gr0, sh);
+        }
     }
     if (G.replay) {
         atomicAdd(G.replay + p * 3, rep.x);
