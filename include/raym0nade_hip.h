@@ -473,7 +473,7 @@ enum rm_tune_key {
     RM_TUNE_TRACE_VARIANT = 0,          /* 0 stack walk (one ray per lane), 2 persistent step walk,
                                            3 persistent walk with its stack in LDS (default; in a render
                                            launch: every walk of its kernels): with RM_TUNE_TRIS_PER_STEP
-                                           0 the walk of a four-wide tree (scenes of at most 48 triangles
+                                           0 the walk of a four-wide tree (scenes of at most 64 triangles
                                            are tested without a tree), else the step walk of the binary
                                            tree; 1 and 4 (a one-ray step walk and two walks per lane) are
                                            retired and rejected */

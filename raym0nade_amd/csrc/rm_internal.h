@@ -168,6 +168,9 @@ namespace rm {
 // Box-filtered mip levels 1.. of texture `t` from its level 0 in the device
 // texel pool, the same arithmetic as the host build (stream-ordered).
 int32_t launch_mip_build(const rm_scene *s, int t, hipStream_t st);
+// Puts a small scene's rejection records (wide.h) behind its triangles;
+// returns their offset in bytes, 0 for other scenes.
+size_t append_flat(HostScene &h);
 // The four-wide tree of an uploaded scene (wide.h); waits for it.
-int32_t build_wide(rm_scene *s);
+int32_t build_wide(rm_scene *s, size_t flat);
 }  // namespace rm

@@ -56,6 +56,15 @@ struct alignas(64) WideNode {
 };
 static_assert(sizeof(WideNode) == 64, "WideNode is one cache line");
 
+// Rejection record of one triangle of a flat scene (wide.h): with a line's
+// direction d and moment m = o x d, Moeller-Trumbore's unscaled values are
+//   a = -n.d,  u a = e2.m + w2.d,  v a = -(e1.m + w1.d)
+// n = e1 x e2, w1 = v0 x e1, w2 = v0 x e2; k scales their error bound.
+struct alignas(64) FlatTri {
+    float e1[3], e2[3], w1[3], w2[3], n[3], k;
+};
+static_assert(sizeof(FlatTri) == 64, "one scalar load");
+
 // Walk-stack capacity: pending entries <= tree depth - 1 (2^27 faces -> 25).
 constexpr int MAX_STACK = 32;
 
@@ -150,6 +159,8 @@ struct SceneView {
     // its coordinates are (x - wide_lo) * wide_scale, a power of two
     const WideNode *wide;
     int32_t flat;                 // the number of triangles when rays test them all (wide.h), else 0
+    float flat_b;                 // three times the largest coordinate of a flat scene
+    const FlatTri *flat_tris;
     float wide_lo[3], wide_scale, wide_rscale;
 };
 

@@ -895,7 +895,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         if (wide) {
             // every wave a few rays, or the whole machine
             const uint32_t most = (uint32_t)device_cu_count() * T.persistent_blocks_per_cu * (TRACE_BLOCK / 64);
-            const uint32_t per = s->view.flat ? 64u : wide_per_wave((uint32_t)n, most);
+            const uint32_t per = wide_per_wave((uint32_t)n, most, s->view.flat);
             const uint32_t waves = (uint32_t)std::min<int64_t>(most, (n + per - 1) / per);
             pgrid = (waves + TRACE_BLOCK / 64 - 1) / (TRACE_BLOCK / 64);
             hipLaunchKernelGGL(k_trace_wide<ANY>, dim3(pgrid), dim3(TRACE_BLOCK), wide_lds_bytes(s->view.depth), st,

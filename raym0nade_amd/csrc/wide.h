@@ -390,21 +390,42 @@ struct RefWalker {
 
 };
 
-// Scenes of at most FLAT_MAX triangles are not walked: every lane tests
-// every triangle, whose record the wave loads once into scalar registers.
-// No lane waits for memory or for lanes at other nodes: a 36-triangle scene's
-// extension rays (2M in a launch) took 285 us in the binary walk, 299 in the
-// wide one and 187 here, a launch of 20k rays 109, 123 and 15.  With the
-// certificate of the wide walk the result is the reference's; a scene of one
-// leaf is tested in the reference's own order.
-constexpr int FLAT_MAX = 48;
+// Scenes of at most FLAT_MAX triangles are not walked.  Every lane passes over
+// every triangle, whose rejection record the wave loads once into scalar
+// registers, and keeps those its line may pass through as a bit mask; then
+// each lane tests its own few with the reference's arithmetic, in order.  No
+// lane waits for lanes at other nodes.  With the certificate of the wide walk
+// the result is the reference's; a scene of one leaf is tested in the
+// reference's own order.
+//
+// The rejection works on the unscaled values a, u a and v a from the line's
+// moment (25 instructions a triangle, the exact test takes 66).  Its own
+// roundings and those of the exact test, whose accepted u and v may lie
+// outside [0, 1] by theirs, stay below 16 eps |d| (|e1| + |e2|) (|o| + |v0| +
+// |e1|) each; twice their sum is allowed (FLAT_ERR, eps = 2^-24).
+//
+// FLAT_MAX is the masks' width.  Closest hits of 2M rays among 12 / 36 / 64
+// triangles take 41 / 80 / 125 us, in the binary walk 616 / 645 / 681, of 20k
+// rays 14 / 14 / 19 and 78 / 97 / 118; 100 triangles in the four-wide tree
+// 439 and 39.  Extension rays of a 512 x 512 Cornell render (36 triangles, 16
+// launches) took 2.99 ms with every triangle tested exactly, 1.00 with the
+// masks and wide_per_wave's shares.
+constexpr int FLAT_MAX = 64;
+constexpr double FLAT_ERR = 64.0 / 16777216.0;
 
 template <bool ANY>
 __device__ __forceinline__ void flat_tris(const SceneView &S, V3 o, V3 d, float tmin, float aim, float &tmax, float &t2,
                                           int32_t &best) {
     typedef const __attribute__((address_space(4))) float scalar_float;
+    const V3 m{__builtin_fmaf(o.y, d.z, -(o.z * d.y)), __builtin_fmaf(o.z, d.x, -(o.x * d.z)),
+               __builtin_fmaf(o.x, d.y, -(o.y * d.x))};
+    const float d1 = (fabsf(d.x) + fabsf(d.y)) + fabsf(d.z);
+    float rho = -d1 * (((fabsf(o.x) + fabsf(o.y)) + fabsf(o.z)) + S.flat_b);
+    // lines whose products could leave the normal numbers keep every triangle
+    if (!(d1 > 1e-5f && rho > -1e18f)) rho = -INFINITY;
+    uint32_t mask[2] = {0u, 0u};
     // one scene at a time: the lanes of a batch may hold several
-    const uint64_t p = (uint64_t)S.tris;
+    const uint64_t p = (uint64_t)S.flat_tris;
     uint64_t pending = __ballot(true);
     while (pending) {
         const int lead = (int)__ffsll((unsigned long long)pending) - 1;
@@ -415,16 +436,40 @@ __device__ __forceinline__ void flat_tris(const SceneView &S, V3 o, V3 d, float 
         const bool mine = p == q;
         if (mine) {
             scalar_float *T = (scalar_float *)q;
-            for (uint32_t i = 0; i < n; ++i, T += sizeof(TriRec) / 4) {
-                const float t = tri_test_flat(o, d, V3{T[0], T[1], T[2]}, T[3], V3{T[4], T[5], T[6]}, V3{T[8], T[9], T[10]});
-                const bool in = tmin < t && t < t2, first = t < tmax;
-                t2 = in ? (first ? tmax : t) : t2;
-                best = in && first ? (int32_t)i : best;
-                tmax = in && first ? t : tmax;
-                if (ANY && !__ballot(!(tmax < aim))) break;
+            for (uint32_t i = 0; i < n; ++i, T += sizeof(FlatTri) / 4) {
+                // -a, u a and -v a of the line; a's sign makes them comparable
+                const float a = __builtin_fmaf(T[12], d.x, __builtin_fmaf(T[13], d.y, T[14] * d.z));
+                const float u = __builtin_fmaf(T[3], m.x, __builtin_fmaf(T[4], m.y, __builtin_fmaf(T[5], m.z,
+                                __builtin_fmaf(T[9], d.x, __builtin_fmaf(T[10], d.y, T[11] * d.z)))));
+                const float v = __builtin_fmaf(T[0], m.x, __builtin_fmaf(T[1], m.y, __builtin_fmaf(T[2], m.z,
+                                __builtin_fmaf(T[6], d.x, __builtin_fmaf(T[7], d.y, T[8] * d.z)))));
+                const uint32_t sg = __float_as_uint(a) & 0x80000000u;
+                const float x = __uint_as_float(__float_as_uint(u) ^ sg ^ 0x80000000u);
+                const float y = __uint_as_float(__float_as_uint(v) ^ sg);
+                const float z = fabsf(a) - (x + y);
+                const bool out = fminf(fminf(x, y), z) < rho * T[15];
+                mask[i >> 5] |= out ? 0u : 1u << (i & 31u);
             }
         }
         pending &= ~__ballot(mine);
+    }
+    while (mask[0] | mask[1]) {
+        uint32_t i;
+        if (mask[0]) {
+            i = (uint32_t)__ffs((int)mask[0]) - 1u;
+            mask[0] &= mask[0] - 1u;
+        } else {
+            i = 31u + (uint32_t)__ffs((int)mask[1]);
+            mask[1] &= mask[1] - 1u;
+        }
+        const TriRec T = load_tri(S.tris, i);
+        const float t = tri_test_flat(o, d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
+                                      V3{T.e2[0], T.e2[1], T.e2[2]});
+        const bool in = tmin < t && t < t2, first = t < tmax;
+        t2 = in ? (first ? tmax : t) : t2;
+        best = in && first ? (int32_t)i : best;
+        tmax = in && first ? t : tmax;
+        if (ANY && tmax < aim) break;
     }
 }
 
@@ -479,7 +524,15 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
 // and 64 each; the walks of a wave wait for each other, and those of many
 // waves compete (closest hits among 1M triangles, 8 / 16 / 32 / 64 rays a
 // wave: 10k rays 223 / 241 / 258 / 278 us, 100k rays 571 / 377 / 344 / 339 us).
-__host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves) {
+// The rays of a flat scene cost the same, so a wave takes whole batches, its
+// whole share at the start where that is at most 512: claims are atomic adds
+// to one address, 12 ns each, and 64 rays a claim held 2M closest hits among
+// 36 triangles to 392 us (80 so, and 302 for 8M).
+__host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bool flat) {
+    if (flat) {
+        const uint32_t p = (n / 64u + waves) / waves * 64u;
+        return p > 512u ? 512u : p;
+    }
     if (n / 64u < waves) {
         const uint32_t p = (uint32_t)(((uint64_t)n * 5u + waves - 1u) / waves);
         return p < 8u ? 8u : p > 64u ? 64u : p;

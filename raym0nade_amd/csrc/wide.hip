@@ -7,6 +7,8 @@
 // node's children sit side by side and every slot is filled by one thread
 // without looking at any other.  A leaf one level above a kept level takes the
 // slot of its first would-be descendant.
+#include <cstring>
+
 #include "rm_internal.h"
 #include "wide.h"
 
@@ -142,23 +144,71 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
                       (uint32_t)org[2] | (half_up(pad_e * scale) << 16), half_up(pad_d * scale), ref);
 }
 
-// Scenes outside the tree's range keep the binary walk: one leaf, 2^25
-// triangles or more (a run's reference), coordinates that are not finite or
-// whose scaling would leave the float range.
-int32_t build_wide(rm_scene *s) {
-    SceneView &v = s->view;
-    v.wide = nullptr;
-    v.flat = 0;
-    const HostScene &h = s->host;
-    if (h.root_leaf) v.flat = (int32_t)h.n;
-    if (h.root_leaf || h.n >= (int64_t(1) << 25)) return RM_OK;
-    float ext = 0.0f, mag = 0.0f;
+// The walks' range: coordinates that are finite and whose scaling stays in
+// the float range.
+static bool wide_range(const HostScene &h, float &ext, float &mag) {
+    ext = mag = 0.0f;
     for (int a = 0; a < 3; ++a) {
-        if (!isfinite(h.root_lo[a]) || !isfinite(h.root_hi[a])) return RM_OK;
+        if (!isfinite(h.root_lo[a]) || !isfinite(h.root_hi[a])) return false;
         ext = std::max(ext, h.root_hi[a] - h.root_lo[a]);
         mag = std::max({mag, fabsf(h.root_lo[a]), fabsf(h.root_hi[a])});
     }
-    if (!(ext > 1e-12f) || !(ext < 1e12f) || mag > 1e4f * ext) return RM_OK;
+    return ext > 1e-12f && ext < 1e12f && mag <= 1e4f * ext;
+}
+
+// A flat scene's records follow its triangles in their buffer: no kernel and
+// no allocation for scenes that are made in half a millisecond.
+size_t append_flat(HostScene &h) {
+    float ext, mag;
+    if (h.n > FLAT_MAX || !wide_range(h, ext, mag)) return 0;
+    const size_t n = (size_t)h.n, off = (n * sizeof(TriRec) + 63) & ~size_t(63);
+    if (!h.root_leaf)  // the leaves' numbers
+        for (uint32_t u = 1; u < h.pairs.size(); ++u)
+            for (uint32_t k = 0; k < 2; ++k)
+                for (uint32_t i = 0; i < (h.pairs[u].leaf[k] & LEAF_MASK); ++i) {
+                    const uint32_t c = 2 * u + k;
+                    std::memcpy(&h.tris[(h.pairs[u].leaf[k] >> LEAF_SHIFT) + i].e2[3], &c, 4);
+                }
+    h.tris.resize((off + n * sizeof(FlatTri) + sizeof(TriRec) - 1) / sizeof(TriRec));
+    for (size_t i = 0; i < n; ++i) {
+        const TriRec T = h.tris[i];
+        double v0[3], e1[3], e2[3], l1 = 0.0, l2 = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            v0[a] = T.p[a], e1[a] = T.e1[a], e2[a] = T.e2[a];
+            l1 += e1[a] * e1[a], l2 += e2[a] * e2[a];
+        }
+        FlatTri F;
+        for (int a = 0; a < 3; ++a) {
+            const int b = (a + 1) % 3, c = (a + 2) % 3;
+            F.e1[a] = T.e1[a], F.e2[a] = T.e2[a];
+            F.w1[a] = (float)(v0[b] * e1[c] - e1[b] * v0[c]);
+            F.w2[a] = (float)(v0[b] * e2[c] - e2[b] * v0[c]);
+            F.n[a] = (float)(e1[b] * e2[c] - e2[b] * e1[c]);
+        }
+        const double len = sqrt(l1) + sqrt(l2);
+        F.k = len > 1e-15 ? (float)(FLAT_ERR * len) : INFINITY;  // shorter, or NaN: never rejected
+        std::memcpy(reinterpret_cast<char *>(h.tris.data()) + off + i * sizeof(FlatTri), &F, sizeof(F));
+    }
+    return off;
+}
+
+// Scenes outside the tree's range keep the binary walk: 2^25 triangles or
+// more (a run's reference), coordinates outside wide_range.  flat: where
+// append_flat put the records, or 0.
+int32_t build_wide(rm_scene *s, size_t flat) {
+    SceneView &v = s->view;
+    v.wide = nullptr;
+    v.flat = 0;
+    v.flat_tris = nullptr;
+    const HostScene &h = s->host;
+    float ext, mag;
+    if (h.n >= (int64_t(1) << 25) || !wide_range(h, ext, mag)) return RM_OK;
+    if (flat) {
+        v.flat = (int32_t)h.n;
+        v.flat_b = 3.0f * mag;
+        v.flat_tris = reinterpret_cast<const FlatTri *>(s->tris.as<char>() + flat);
+        return RM_OK;
+    }
     const int e = (int)floor(log2(30000.0 / (double)ext));
     const double scale = ldexp(1.0, e);
     for (int a = 0; a < 3; ++a) v.wide_lo[a] = (float)((double)h.root_lo[a] - 1000.0 / scale);
@@ -174,7 +224,7 @@ int32_t build_wide(rm_scene *s) {
         total += std::max(4u, 1u << l);
         l += step;
     }
-    int32_t rc = s->wide.alloc((size_t)total * sizeof(WideNode));
+    const int32_t rc = s->wide.alloc((size_t)total * sizeof(WideNode));
     if (rc) return rc;
     for (size_t i = 0; i < levels.size(); ++i) {
         const Level &L = levels[i];
@@ -187,7 +237,6 @@ int32_t build_wide(rm_scene *s) {
     // the caller may use the scene on any stream next
     RM_HIP(hipStreamSynchronize(nullptr));
     v.wide = s->wide.as<WideNode>();
-    if (h.n <= FLAT_MAX) v.flat = (int32_t)h.n;
     return RM_OK;
 }
 

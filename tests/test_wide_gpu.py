@@ -1,7 +1,7 @@
 """The four-wide walk and the flat test of small scenes (trace variant 3 with
 whole leaves, the default) against the oracle's BVH::rayHit / Model::rayHit_test: ids, t and
 occlusion bit-exact.  Scenes around the sizes where the tree changes (one
-leaf, 48 / 49 triangles, odd and even numbers of levels, uneven leaves,
+leaf, 64 / 65 triangles, slivers far from the origin, odd and even numbers of levels, uneven leaves,
 duplicated triangles, axis-aligned walls, large triangles among small ones);
 rays aimed at vertices and edges (exact ties and certificates that fail), from
 surfaces, along axes exactly and nearly, from far outside, of lengths other
@@ -41,6 +41,8 @@ def walls(n):
 SCENES = {
     "one_leaf": lambda: soup(10, 1, 0.5), "two_leaves": lambda: soup(11, 2, 0.5), "soup20": lambda: soup(20, 3, 0.4),
     "soup21": lambda: soup(21, 4, 0.4), "soup48": lambda: soup(48, 5, 0.3), "soup49": lambda: soup(49, 6, 0.3),
+    "soup64": lambda: soup(64, 13, 0.3), "soup65": lambda: soup(65, 14, 0.3),
+    "slivers": lambda: (soup(60, 15, 0.8) * np.array([1, 1e-4, 1]) + np.array([90, 40, -7])).astype(np.float32),
     "soup80": lambda: soup(80, 7, 0.3), "soup81": lambda: soup(81, 8, 0.3), "soup1301": lambda: soup(1301, 9),
     "soup7001": lambda: soup(7001, 10, 0.05), "walls": lambda: walls(9),
     "doubled": lambda: np.repeat(soup(700, 11, 0.2), 2, axis=0),
@@ -108,10 +110,11 @@ def test_bit_exact(dev, scene):
         assert np.array_equal(occ.cpu().numpy(), OS.any(r, aims=aim)), (scene, kind)
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 511, 1639, 13107, 131073])
-def test_ray_counts(dev, n):
+@pytest.mark.parametrize("tris", [36, 3001])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 511, 1639, 13107, 131073, 524287, 4194305])
+def test_ray_counts(dev, n, tris):
     """Every split of a batch over waves and lanes gives the reference walk's results."""
-    S = rm.Scene(rm.generate(1, 5, n_tris=3001))
+    S = rm.Scene(rm.generate(1, 5, n_tris=tris))
     r = torch.from_numpy(rm.rays(1, n, seed=n)).to(dev)
     t, ids = S.trace_closest(r)
     occ = S.trace_any(r, aim=0.3)
