@@ -495,12 +495,15 @@ enum rm_tune_key {
     RM_TUNE_RENDER_MIN_WAVES = 7,       /* 1 (default), 3 or 4: resident waves per SIMD the render's
                                            shading and NEE kernels are compiled for (3 caps them
                                            at 168 VGPRs, 4 at 128, spilling the rest) */
-    RM_TUNE_LDS_STACK_ENTRIES = 8,      /* trace variant 3: walk-stack entries per lane kept in LDS
-                                           (1..32, default 10: 160 KiB of LDS at 8 blocks/CU; deeper
+    RM_TUNE_LDS_STACK_ENTRIES = 8,      /* trace variant 3's walk of the binary tree (the four-wide walk
+                                           sizes its own): walk-stack entries per lane kept in LDS (1..32, default 10: 160 KiB of LDS at 8 blocks/CU; deeper
                                            entries go to scratch; 32 holds the whole stack of any tree) */
-    RM_TUNE_TRIS_PER_STEP = 9           /* trace variant 3 and render walks: triangles one walk step
-                                           tests (0 = a whole leaf (default); 1, 2 or 4: a leaf over
-                                           several steps; the render's shading kernels use 0 or 2) */,
+    RM_TUNE_TRIS_PER_STEP = 9           /* trace variant 3 and render walks: 0 (default) the walk of the
+                                           four-wide tree; 1, 2 or 4: the binary tree's, that many
+                                           triangles of a leaf tested a step (the render's shading
+                                           kernels use 2).  Where the four-wide walk does not apply
+                                           (utilisation or render counts on, scenes outside its range)
+                                           0 is the binary tree's with whole leaves */,
     RM_TUNE_NEE_SPLIT = 10,             /* render: 1 traces the shadow rays of light samples (the
                                            primary vertex's and the NEE records') in their own
                                            persistent passes, 0 inside the sampling kernels, 2 (default)
