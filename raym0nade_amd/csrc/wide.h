@@ -530,7 +530,7 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
 // 36 triangles to 392 us (80 so, and 302 for 8M).
 __host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bool flat) {
     if (flat) {
-        const uint32_t p = (n / 64u + waves) / waves * 64u;
+        const uint32_t p = ((n - 1u) / 64u + waves) / waves * 64u;
         return p > 512u ? 512u : p;
     }
     if (n / 64u < waves) {
