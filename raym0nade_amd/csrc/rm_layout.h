@@ -48,9 +48,11 @@ static_assert(sizeof(TriRec) == 48, "TriRec is 48 B");
 // planes (four fp16, two words) then their upper planes, as offsets from the
 // node's origin in scaled coordinates; an empty child has an infinite lower
 // and a zero upper plane.  m[0] = origin x | y << 16, m[1] = origin z | E << 16,
-// m[2] = D (fp16), m[3] = reference of child 0 (child k: + k).  E and D are 0
-// except over the runs of a leaf: the largest |e2| of its triangles and the
-// diagonal of their bounds, scaled, fp16 rounded up.
+// m[2] = D | all << 16 | flags << 28, m[3] = reference of child 0 (child k: + k).
+// E: the largest |e2| of the triangles below the children without a flag,
+// scaled; D: the distance from the origin to the farthest corner of the
+// children; both fp16 rounded up.  Flag k: child k holds larger triangles.
+// all: the largest |e2| of all triangles below, an fp16 number's upper 12 bits.
 struct alignas(64) WideNode {
     uint32_t x[4], y[4], z[4], m[4];
 };
@@ -162,6 +164,9 @@ struct SceneView {
     float flat_b;                 // three times the largest coordinate of a flat scene
     const FlatTri *flat_tris;
     float wide_lo[3], wide_scale, wide_rscale;
+    float wide_mid[3], wide_reach;  // where most triangles lie, in these coordinates: around, how far apart
+    int32_t n_big;                // much larger triangles, tested before the walk: their slots
+    const uint32_t *big;
 };
 
 }  // namespace rm

@@ -7,17 +7,30 @@
 // running t_max), the reference visits a leaf for certain when G holds and L
 // lies below its running t_max: the boxes of the leaf's ancestors contain the
 // leaf's, and every operation of the slab test is monotone, so theirs pass
-// too.  Hence, if a walk that misses no leaf the reference could visit ends
-// with closest hit t* in one leaf, every other accepted t being >= t2, then
-//     G(leaf)  and  t* < t2  and  L(leaf) < t2
+// too.  Let a walk end with closest hit t* in one leaf, t2 being the least t
+// it accepted in other leaves, and let no triangle that it did not test have a
+// computed t below lim(t*), somewhat more than t*.  Then
+//     G(leaf)  and  t* < t2  and  L(leaf) < min(t2, lim(t*))
 // proves that the reference ends with the same triangle: its t_max stays
-// >= t2 until it reaches that leaf.  The walk here tests a superset of the
+// >= min(t2, lim(t*)) until it reaches that leaf, and > t* then, and later
+// hits are no closer.  The walk here tests a superset of the
 // reference's boxes with cheap arithmetic (fused multiply-adds on 16-bit
 // boxes, rounded outward, with margins that cover every rounding) and checks
 // this certificate once per ray, on the reference's own box.  Where it fails
 // -- two hits within a rounding error of each other -- the ray is walked
-// again in the reference's order, by the same lane (RefWalker).  A shadow ray is blocked for
-// certain when an accepted t < aim lies in a leaf with G and L < aim.
+// again in the reference's order, by the same lane (RefWalker).  A shadow ray
+// is blocked for certain when an accepted t < aim lies in a leaf with G and
+// L < aim.
+//
+// What the walk leaves out lies beyond the closest hit so far by its box.  But
+// the computed t of a triangle that the ray grazes can lie far before the box
+// that holds the triangle, so boxes are grown by a bound of that error
+// (WIDE_ERR) from the largest edge among the triangles below a node.  A
+// triangle much larger than those around it would grow every box up to the
+// root by its own edge.  A few such triangles (a ground, the walls of a room)
+// are tested before the walk and left out of the growth; where there are more,
+// they leave the others' bounds as they are, and the children on the way to
+// them are flagged and always entered.
 //
 // Node, 64 B (a cache line), four children: origin on a 16-bit grid, child
 // boxes as offsets from it in fp16, so a box plane costs one mixed-precision
@@ -32,12 +45,14 @@
 // incoherent 1M-triangle batch it spent 8.1 ms with the vector ALUs issuing
 // 87% of the time and the texture data path busy 97% of it: every 16 bytes a
 // lane loads occupies that path for a cycle of its compute unit, and a ray
-// loaded 511 of them (88 nodes of 64 B, 61 triangles of 48 B).  Here it loads
-// 287 (46 nodes, 18 runs), and 44 of a wave's 64 lanes take part in a node's
-// step instead of 30.  Before and after (us, launches included): 8M incoherent
-// rays 8560 -> 4820, 8M camera rays 3440 -> 2660, 100k incoherent rays among
-// 200k triangles 583 -> 330, 1M shadow rays 1013 -> 704; 1080p frame of 2M
-// triangles at 16 spp 154 -> 116 ms.  What bounds it now: the same data path
+// loaded 511 of them (88 nodes of 64 B, 61 triangles of 48 B).  Here, before
+// boxes were grown, it loaded 287 (46 nodes, 18 runs), and 44 of a wave's 64
+// lanes took part in a node's step instead of 30.  Before and after (us,
+// launches included): 8M incoherent rays 8560 -> 4940, 8M camera rays 3440 ->
+// 2865, 100k incoherent rays among 200k triangles 583 -> 335, 1M shadow rays
+// 1013 -> 700; 1080p frame of 2M triangles at 16 spp 154 -> 114 ms.  (The growth
+// takes 3 to 5% of these batches; without the list of large triangles it took
+// 10% of scenes of small spheres on a ground.)  What bounds it now: the same data path
 // (94% busy), then the vector ALUs.
 #pragma once
 #include <type_traits>
@@ -87,22 +102,41 @@ struct WideRay {
     V3 o, d;         // as given: the triangle tests use these
     float inv[3];
     float nr[3], fr[3];
-    float scale;     // scene units to scaled ones
-    float err;       // WIDE_ERR |d| / scale, negative for a ray with parallel axes
+    float err;       // WIDE_ERR |d| / scale: a box grows by err E distance; negative for a ray with parallel axes
 };
 
-// Displacement of a triangle test's accepted region, over |d| |e2| S / scale
-// (S: distance to the triangle): the roundings of u and v each move it by at
-// most 7.5 eps S |d| |e1| |e2| / |a| along an edge and that of a by about as
-// much, and a test with |a| < 1e-4 |e1| is rejected: 2 * 7.5 eps / 1e-4 + the
-// last, eps = 2^-24.
+// How far from a triangle the test accepts a ray: with the computed a, u, v
+// and t of an accepted test, eps = 2^-24 and s = o - v0,
+//     R = s - u e1 - v e2 + t d
+//     a R = da s - du e1 - dv e2 + dt d
+// where da..dt are the errors of the computed e1.h, s.h, d.q and e2.q (Cramer:
+// without them the right side is 0).  A cross product is off by at most (2 /
+// sqrt 3 + 1) eps times its factors' lengths and a dot product by 3 eps more,
+// so each of the four terms is at most 5.16 eps |d| |e1| |e2| |s|; and a test
+// with |a| < 1e-4 |e1| is rejected.  So o + t d, the point where the reference
+// has the hit, lies within |R| <= 4 * 5.16 eps / 1e-4 |d| |e2| |s| = 0.01231
+// |d| |e2| |s| of v0 + u e1 + v e2, a point of the triangle.  (Rounding s, e1
+// and e2 moves it by parts of 1e-7 of the coordinates, which wide_ray's margins
+// cover.)  A box that holds the triangle, grown by that much, is entered no
+// later than at the computed t.
+//
+// The bound grows with the square of a scene's size, and grown boxes are
+// entered more often, so the tree serves scenes and rays of moderate size
+// only, others walk the binary tree.  WIDE_SCENE bounds the growth relative to
+// |e2| over the size of a scene for |d| = 1: over 10 / 30 / 100 units, closest
+// hits among a million triangles take 0.57 / 0.73 / 1.33 of the binary walk's
+// time, 5000 take 0.65 / 0.88 / 1.75, 300 take 0.70 / 1.04 / 1.64.  WIDE_FAR bounds it for a
+// ray, which RefWalker serves otherwise, more slowly than the binary walk's
+// kernels: at 1.3 the grown boxes take 1.1 to 1.9 of those kernels' time.
 constexpr float WIDE_ERR = 0.0126f;
+constexpr float WIDE_SCENE = 0.4f, WIDE_FAR = 1.5f;
 // The entry distances' slack below the running t_max: 3 eps_zero of rayInBox,
 // rounding and a margin.
 __device__ __forceinline__ float wide_limit(float t) { return __builtin_fmaf(fabsf(t), 0x1p-16f, t) + 4.2e-4f; }
 
 // Sets up the ray; false when it is outside the margins' range (origin far
-// outside the scene, non-finite or extreme values, a negative tmin): such rays are walked in the reference's order.
+// outside the scene, non-finite or extreme values, a negative tmin) or
+// WIDE_FAR: such rays are walked in the reference's order.
 __device__ __forceinline__ bool wide_ray(const SceneView &S, V3 o, V3 d, float tmin, WideRay &r) {
     r.o = o;
     r.d = d;
@@ -110,12 +144,13 @@ __device__ __forceinline__ bool wide_ray(const SceneView &S, V3 o, V3 d, float t
                         (o.z - S.wide_lo[2]) * S.wide_scale};
     const float dv[3] = {d.x, d.y, d.z};
     const float far = fmaxf(fmaxf(fabsf(p[0]), fabsf(p[1])), fabsf(p[2]));
+    const float off = fmaxf(fmaxf(fabsf(p[0] - S.wide_mid[0]), fabsf(p[1] - S.wide_mid[1])), fabsf(p[2] - S.wide_mid[2]));
     const float dmax = fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z));
     // fmax drops NaNs, so they are looked for in the sums
     const float sum = ((p[0] + p[1]) + p[2]) + ((d.x + d.y) + d.z);
-    const bool ok = tmin >= 0.0f && far < 4e6f && dmax > 1e-3f && dmax < 1e9f && sum == sum;
-    r.scale = S.wide_scale;
-    r.err = (fabsf(d.x) + fabsf(d.y) + fabsf(d.z)) * S.wide_rscale * WIDE_ERR;
+    r.err = length(d) * S.wide_rscale * WIDE_ERR;
+    const bool ok = tmin >= 0.0f && far < 4e6f && dmax > 1e-3f && dmax < 1e9f && sum == sum &&
+                    r.err * (off + S.wide_reach) < WIDE_FAR;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const bool par = fabsf(dv[k]) < T_EPS;
@@ -221,8 +256,7 @@ struct WideWalker {
     // visits a leaf only when the origin lies within its box, so the distance
     // there is at most the leaf's size (D once more); and over the runs, which
     // are smaller than the leaf, the ray drifts by its small component.
-    static __device__ __forceinline__ float par_pad(const WideRay &r, const float (&cn)[3], uint4 M) {
-        if (!(M.w & 0x80000000u)) return 0.0f;
+    static __device__ __forceinline__ float par_pad(const WideRay &r, float scale, const float (&cn)[3], uint4 M) {
         const float d[3] = {fabsf(r.d.x), fabsf(r.d.y), fabsf(r.d.z)};
         float sum = 0.0f, drift = 0.0f;
 #pragma unroll
@@ -231,12 +265,13 @@ struct WideWalker {
             sum += par ? 0.0f : fabsf(cn[a]) * d[a];
             drift = par ? fmaxf(drift, d[a]) : drift;
         }
-        const float dist = __builtin_fmaf(sum, r.scale, 2.0f * half_lo(M.z));
-        return (drift / fmaxf(fmaxf(d[0], d[1]), d[2]) - r.err * half_hi(M.y)) * dist;
+        const float dist = __builtin_fmaf(sum, scale, 2.0f * half_lo(M.z));
+        const float pad = -r.err * half_hi(M.y) * dist;
+        return M.w & 0x80000000u ? __builtin_fmaf(drift / fmaxf(fmaxf(d[0], d[1]), d[2]), dist, pad) : pad;
     }
 
     // Visits cur.
-    __device__ __forceinline__ void step_node(const WideNode *nodes, const WideRay &r, float tmin) {
+    __device__ __forceinline__ void step_node(const WideNode *nodes, float scale, const WideRay &r, float tmin) {
         const float lim = wide_limit(tmax);
         const uint4 *P = reinterpret_cast<const uint4 *>(nodes + cur);
         const uint4 X = P[0], Y = P[1], Z = P[2], M = P[3];
@@ -249,18 +284,21 @@ struct WideWalker {
             cf[a] = __builtin_fmaf(org[a], r.inv[a], r.fr[a]);
             sg[a] = (uint32_t)((int32_t)__float_as_uint(r.inv[a]) >> 31);
         }
-        // over a leaf's runs: how far a triangle's accepted region may reach
-        // beyond it, from this distance (at most that to the node's origin
-        // along the axes, plus D)
-        const float dist = __builtin_fmaf(__builtin_fmaf(fabsf(cn[0]), fabsf(r.d.x),
-                                                         __builtin_fmaf(fabsf(cn[1]), fabsf(r.d.y), fabsf(cn[2]) * fabsf(r.d.z))),
-                                          r.scale, half_lo(M.z));
+        // how far from a triangle below the ray may pass where the test
+        // accepts it (WIDE_ERR): at this distance, at most that to the node's
+        // origin along the axes, plus D.  Entries are that much earlier; over
+        // a leaf's runs, which the reference does not test, exits later too.
+        const float dx = fabsf(cn[0] * r.d.x), dy = fabsf(cn[1] * r.d.y), dz = fabsf(cn[2] * r.d.z);
+        // (a 2-norm is at most 0.415 times the sum and 0.585 times the largest)
+        const float dist = __builtin_fmaf(__builtin_fmaf(0.585f, fmaxf(fmaxf(dx, dy), dz), 0.415f * (dx + dy + dz)), scale, half_lo(M.z));
         float pad = r.err * half_hi(M.y) * dist;
-        if (r.err < 0.0f) pad = par_pad(r, cn, M);
+        if (r.err < 0.0f) pad = par_pad(r, scale, cn, M);
+        pad = fminf(pad, 1e9f);  // an infinite E: beyond every coordinate
+        const float padf = __uint_as_float(__float_as_uint(pad) & (uint32_t)((int32_t)M.w >> 31));
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             cn[a] = __builtin_fmaf(-pad, fabsf(r.inv[a]), cn[a]);
-            cf[a] = __builtin_fmaf(pad, fabsf(r.inv[a]), cf[a]);
+            cf[a] = __builtin_fmaf(padf, fabsf(r.inv[a]), cf[a]);
         }
         const uint32_t nx[2] = {bit_select(sg[0], X.z, X.x), bit_select(sg[0], X.w, X.y)};
         const uint32_t fx[2] = {bit_select(sg[0], X.x, X.z), bit_select(sg[0], X.y, X.w)};
@@ -285,6 +323,14 @@ struct WideWalker {
             const uint32_t e = en <= ex ? __float_as_uint(en) : 0x7f800000u;
             key[k] = (int)((e & ~3u) | (uint32_t)k);
         }
+        // children with larger triangles are entered whatever E says, after
+        // the others where their boxes say no
+        const uint32_t flags = M.z >> 28;
+        if (flags) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (flags & (1u << k)) key[k] = key[k] < 0x7f7ffffc ? key[k] : 0x7f7ffffc | k;
+        }
         // sort the four, nearest first
 #define RM_CSWAP(a, b)                                  \
     {                                                   \
@@ -304,10 +350,33 @@ struct WideWalker {
         if (n) {
             if (gy) stk.put(sp++, gx, gy);
             gx = M.w;
-            gy = ((uint32_t)key[0] & GROUP_T) | n | ((uint32_t)key[0] & 3u) | ((uint32_t)key[1] & 3u) << 2 |
+            gy = (flags ? 0u : (uint32_t)key[0] & GROUP_T) | n | ((uint32_t)key[0] & 3u) | ((uint32_t)key[1] & 3u) << 2 |
                  ((uint32_t)key[2] & 3u) << 4 | ((uint32_t)key[3] & 3u) << 6;
         }
         next(lim);
+    }
+
+    // Tests a triangle (twice is as good as once).
+    __device__ __forceinline__ void test(const TriRec *tris, uint32_t i, V3 o, V3 d, float tmin) {
+        TriRec T = load_tri(tris, i);
+        // the whole record at once: v0 loaded past the first rejection
+        // would cost a second memory latency
+        asm volatile("" : "+v"(T.p[0]), "+v"(T.p[1]), "+v"(T.p[2]));
+        const float t = tri_test_flat(o, d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
+                                      V3{T.e2[0], T.e2[1], T.e2[2]});
+        if (tmin < t && t < t2) {
+            if (t < tmax) {
+                t2 = tmax;
+                tmax = t;
+                best = (int32_t)i;
+            } else if (best != (int32_t)i) {
+                t2 = t;
+            }
+        }
+    }
+    // Those that the boxes' growth leaves out.
+    __device__ __forceinline__ void test_big(const SceneView &S, V3 o, V3 d, float tmin) {
+        for (int k = 0; k < S.n_big; ++k) test(S.tris, S.big[k], o, d, tmin);
     }
 
     // Tests the first run of l.
@@ -315,21 +384,7 @@ struct WideWalker {
         const uint32_t first = (lx >> 6) & 0x1ffffffu, c = (lx >> 2) & 15u, k = ly & 3u;
         const uint32_t end = first + (c * (k + 1u) >> 2);
         for (uint32_t i = first + (c * k >> 2); i < end; ++i) {
-            TriRec T = load_tri(tris, i);
-            // the whole record at once: v0 loaded past the first rejection
-            // would cost a second memory latency
-            asm volatile("" : "+v"(T.p[0]), "+v"(T.p[1]), "+v"(T.p[2]));
-            const float t = tri_test_flat(r.o, r.d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
-                                          V3{T.e2[0], T.e2[1], T.e2[2]});
-            if (tmin < t && t < t2) {
-                if (t < tmax) {
-                    t2 = tmax;
-                    tmax = t;
-                    best = (int32_t)i;
-                } else {
-                    t2 = t;
-                }
-            }
+            test(tris, i, r.o, r.d, tmin);
         }
         drop_first(ly);
         const float lim = wide_limit(tmax);
@@ -494,12 +549,13 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
     if (S.flat) {
         flat_tris<ANY>(S, o, d, tmin, aim, w.tmax, w.t2, w.best);
     } else if (S.wide && wide_ray(S, o, d, tmin, r)) {
-        while (true) {
+        w.test_big(S, o, d, tmin);
+        while (!(ANY && w.tmax < aim)) {
             if (w.has_run()) {
                 w.step_run(S.tris, r, tmin);
                 if (ANY && w.tmax < aim) break;
             } else if (w.has_node()) {
-                w.step_node(S.wide, r, tmin);
+                w.step_node(S.wide, S.wide_scale, r, tmin);
             } else {
                 break;
             }
@@ -618,6 +674,9 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
                         in_ref = true;
                         ref.init((uint32_t)S.root_leaf);
                         w.stop();
+                    } else {
+                        w.test_big(S, o, d, tmin);
+                        if (ANY && w.tmax < aim) w.stop();
                     }
                 }
             }
@@ -641,7 +700,8 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
                 if (ANY && w.tmax < aim) w.stop();
             }
         } else if (w.has_node()) {
-            w.step_node(src.scene().wide, r, tmin);
+            const SceneView &S = src.scene();
+            w.step_node(S.wide, S.wide_scale, r, tmin);
         }
     }
 }

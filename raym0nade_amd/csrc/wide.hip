@@ -7,6 +7,7 @@
 // node's children sit side by side and every slot is filled by one thread
 // without looking at any other.  A leaf one level above a kept level takes the
 // slot of its first would-be descendant.
+#include <algorithm>
 #include <cstring>
 
 #include "rm_internal.h"
@@ -14,7 +15,9 @@
 
 namespace rm {
 
-// fp16 bits of v >= 0 rounded down or up (up: at most 65504).
+constexpr uint32_t MAX_BIG = 8;
+
+// fp16 bits of v >= 0 rounded down or up (up: at most 65504, or infinity).
 __device__ __forceinline__ uint32_t half_down(double v) {
     if (!(v > 0.0)) return 0u;
     const _Float16 h = (_Float16)v;
@@ -24,6 +27,7 @@ __device__ __forceinline__ uint32_t half_down(double v) {
 }
 __device__ __forceinline__ uint32_t half_up(double v) {
     if (!(v > 0.0)) return 0u;
+    if (v == INFINITY) return 0x7c00u;
     const _Float16 h = (_Float16)v;
     uint32_t b = __builtin_bit_cast(unsigned short, h);
     if (b >= 0x7bffu) return 0x7bffu;
@@ -44,10 +48,31 @@ __device__ void set_child(WideBoxes &B, int k, const PairNode &P, int side) {
     B.used[k] = true;
 }
 
+// A node's E from its children's v: a child whose triangles are much larger
+// than its siblings', so that the growth at the scene's size would show beside
+// the node's own (`size`), is flagged instead.
+__device__ __forceinline__ uint32_t flag_children(const double (&v)[4], const bool (&used)[4], double size, double reach,
+                                                  double &e) {
+    double least = INFINITY;
+    for (int k = 0; k < 4; ++k)
+        if (used[k]) least = fmin(least, v[k]);
+    uint32_t flags = 0u;
+    e = 0.0;
+    for (int k = 0; k < 4; ++k) {
+        if (!used[k]) continue;
+        if (v[k] > 4.0 * least && WIDE_ERR * v[k] * reach > size * 0.0625)
+            flags |= 1u << k;
+        else
+            e = fmax(e, v[k]);
+    }
+    return flags;
+}
+
 __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__ bin, TriRec *__restrict__ tris,
                                                     const TriShade *__restrict__ shade, WideNode *__restrict__ out,
                                                     uint32_t off, int level, int step, uint32_t child_off, float lx,
-                                                    float ly, float lz, double scale) {
+                                                    float ly, float lz, double scale, double reach, double big,
+                                                    uint32_t *__restrict__ found) {
     const uint32_t j = blockIdx.x * 256 + threadIdx.x;
     if (j >= (1u << level)) return;
     // what heap node w = 2^level + j is: follow its bits from the root
@@ -65,13 +90,12 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
     if (leaf && (b > 1 || (b == 1 && (w & 1u)))) return;
     WideBoxes B;
     for (int k = 0; k < 4; ++k) B.used[k] = false;
-    double pad_e = 0.0, pad_d = 0.0;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};  // the largest |e2| below each child, scaled
     uint32_t ref;
     const float lo[3] = {lx, ly, lz};
     if (leaf) {
         const uint32_t first = leaf >> LEAF_SHIFT, c = leaf & LEAF_MASK;
         ref = 0x80000000u | (first << 6) | (c << 2);
-        float all_lo[3] = {INFINITY, INFINITY, INFINITY}, all_hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (uint32_t k = 0; k < 4; ++k) {
             for (int a = 0; a < 3; ++a) {
                 B.lo[k][a] = INFINITY;
@@ -84,22 +108,24 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
                         B.lo[k][a] = fminf(B.lo[k][a], x);  // a NaN is dropped: its triangle is never hit
                         B.hi[k][a] = fmaxf(B.hi[k][a], x);
                     }
-                const double ex = tris[i].e2[0], ey = tris[i].e2[1], ez = tris[i].e2[2];
-                pad_e = fmax(pad_e, sqrt(ex * ex + ey * ey + ez * ez));
+                double l1 = 0.0, l2 = 0.0;
+                for (int a = 0; a < 3; ++a) {
+                    l1 += (double)tris[i].e1[a] * tris[i].e1[a];
+                    l2 += (double)tris[i].e2[a] * tris[i].e2[a];
+                }
+                // (|e1|'s square may leave the float range in the reference's
+                // rejection, which then bounds nothing)
+                const double l = l1 > 1e-30 || l1 == 0.0 ? sqrt(l2) : INFINITY;
+                if (l > big) {  // found[0] of them, the first ones' slots behind
+                    const uint32_t q = atomicAdd(found, 1u);
+                    if (q < MAX_BIG) found[1 + q] = i;
+                } else {
+                    v[k] = fmax(v[k], l * scale);
+                }
                 tris[i].e2[3] = __uint_as_float(u);
             }
             // (a run without triangles keeps its inverted bounds)
             B.used[k] = B.lo[k][0] <= B.hi[k][0] && B.lo[k][1] <= B.hi[k][1] && B.lo[k][2] <= B.hi[k][2];
-            if (B.used[k])
-                for (int a = 0; a < 3; ++a) {
-                    all_lo[a] = fminf(all_lo[a], B.lo[k][a]);
-                    all_hi[a] = fmaxf(all_hi[a], B.hi[k][a]);
-                }
-        }
-        if (all_lo[0] <= all_hi[0]) {
-            const double dx = (double)all_hi[0] - all_lo[0], dy = (double)all_hi[1] - all_lo[1],
-                         dz = (double)all_hi[2] - all_lo[2];
-            pad_d = 1.3 * sqrt(dx * dx + dy * dy + dz * dz);  // distance to v0, and the share of |e1| in the a term
         }
     } else {
         const uint32_t cj = step == 1 ? 2u * j : 4u * j;
@@ -116,6 +142,9 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
                 set_child(B, 2 * s + 1, Q, 1);
             }
         }
+        for (int k = 0; k < 4; ++k)  // (the upper bits of an fp16 number)
+            if (B.used[k])
+                v[k] = (double)__builtin_bit_cast(_Float16, (unsigned short)((out[ref + k].m[2] >> 16 & 0xfffu) << 3));
     }
     double org[3];
     for (int a = 0; a < 3; ++a) {
@@ -136,12 +165,22 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
         pl[a][2] = h[0] | (h[1] << 16);
         pl[a][3] = h[2] | (h[3] << 16);
     }
+    // D: from the node's origin to the farthest corner of its children, and
+    // one unit more for the roundings of a walk's distance to that origin
+    double far[3] = {0.0, 0.0, 0.0};
+    for (int a = 0; a < 3; ++a)
+        for (int k = 0; k < 4; ++k)
+            if (B.used[k]) far[a] = fmax(far[a], ((double)B.hi[k][a] - lo[a]) * scale - org[a]);
+    const double d = sqrt(far[0] * far[0] + far[1] * far[1] + far[2] * far[2]) + 1.0;
+    double e;
+    const uint32_t flags = flag_children(v, B.used, d, reach, e);
+    const uint32_t all = (half_up(fmax(fmax(v[0], v[1]), fmax(v[2], v[3]))) + 7u) >> 3;
     uint4 *o = reinterpret_cast<uint4 *>(out + (off + j));
     o[0] = make_uint4(pl[0][0], pl[0][1], pl[0][2], pl[0][3]);
     o[1] = make_uint4(pl[1][0], pl[1][1], pl[1][2], pl[1][3]);
     o[2] = make_uint4(pl[2][0], pl[2][1], pl[2][2], pl[2][3]);
     o[3] = make_uint4((uint32_t)org[0] | ((uint32_t)org[1] << 16),
-                      (uint32_t)org[2] | (half_up(pad_e * scale) << 16), half_up(pad_d * scale), ref);
+                      (uint32_t)org[2] | (half_up(e) << 16), half_up(d) | (all << 16) | (flags << 28), ref);
 }
 
 // The walks' range: coordinates that are finite and whose scaling stays in
@@ -154,6 +193,35 @@ static bool wide_range(const HostScene &h, float &ext, float &mag) {
         mag = std::max({mag, fabsf(h.root_lo[a]), fabsf(h.root_hi[a])});
     }
     return ext > 1e-12f && ext < 1e12f && mag <= 1e4f * ext;
+}
+
+// Where most triangles lie, whatever a few far ones (a ground) span: the mean
+// of up to 1024 of them and the side of a uniform distribution of their spread.
+// big: BIG_EDGES times their median |e2|.
+constexpr double BIG_EDGES = 16.0;
+static double wide_core(const HostScene &h, double (&mid)[3], double &big) {
+    const int64_t n = std::min<int64_t>(h.n, 1024);
+    double reach = 0.0;
+    for (int a = 0; a < 3; ++a) {
+        double s = 0.0, q = 0.0, m = 0.0;
+        const double c = h.root_lo[a];
+        for (int64_t i = 0; i < n; ++i) {
+            const double x = (double)h.tris[i * h.n / n].p[a] - c;
+            if (!(fabs(x) < 1e30)) continue;
+            s += x, q += x * x, m += 1.0;
+        }
+        mid[a] = c + (m > 0.0 ? s / m : 0.0);
+        if (m > 0.0) reach = std::max(reach, sqrt(std::max(0.0, 12.0 * (q / m - s / m * (s / m)))));
+    }
+    std::vector<float> e((size_t)n);
+    for (int64_t i = 0; i < n; ++i) {
+        const float *v = h.tris[i * h.n / n].e2;
+        const float q = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+        e[(size_t)i] = q == q ? q : 0.0f;
+    }
+    std::nth_element(e.begin(), e.begin() + n / 2, e.end());
+    big = BIG_EDGES * sqrt((double)e[(size_t)(n / 2)]);
+    return reach;
 }
 
 // A flat scene's records follow its triangles in their buffer: no kernel and
@@ -193,13 +261,16 @@ size_t append_flat(HostScene &h) {
 }
 
 // Scenes outside the tree's range keep the binary walk: 2^25 triangles or
-// more (a run's reference), coordinates outside wide_range.  flat: where
+// more (a run's reference), coordinates outside wide_range, and sizes that
+// WIDE_SCENE excludes.  flat: where
 // append_flat put the records, or 0.
 int32_t build_wide(rm_scene *s, size_t flat) {
     SceneView &v = s->view;
     v.wide = nullptr;
     v.flat = 0;
     v.flat_tris = nullptr;
+    v.n_big = 0;
+    v.big = nullptr;
     const HostScene &h = s->host;
     float ext, mag;
     if (h.n >= (int64_t(1) << 25) || !wide_range(h, ext, mag)) return RM_OK;
@@ -209,11 +280,17 @@ int32_t build_wide(rm_scene *s, size_t flat) {
         v.flat_tris = reinterpret_cast<const FlatTri *>(s->tris.as<char>() + flat);
         return RM_OK;
     }
+    double mid[3];
+    double big;
+    const double reach = wide_core(h, mid, big);
+    if (!(WIDE_ERR * reach <= WIDE_SCENE)) return RM_OK;
     const int e = (int)floor(log2(30000.0 / (double)ext));
     const double scale = ldexp(1.0, e);
     for (int a = 0; a < 3; ++a) v.wide_lo[a] = (float)((double)h.root_lo[a] - 1000.0 / scale);
     v.wide_scale = (float)scale;
     v.wide_rscale = (float)(1.0 / scale);
+    for (int a = 0; a < 3; ++a) v.wide_mid[a] = (float)((mid[a] - v.wide_lo[a]) * scale);
+    v.wide_reach = (float)(reach * scale);
     const int leaf_level = h.depth - 1;  // the deepest leaves' level
     struct Level { int level, step; uint32_t off; };
     std::vector<Level> levels;
@@ -224,18 +301,26 @@ int32_t build_wide(rm_scene *s, size_t flat) {
         total += std::max(4u, 1u << l);
         l += step;
     }
-    const int32_t rc = s->wide.alloc((size_t)total * sizeof(WideNode));
+    const int32_t rc = s->wide.alloc((size_t)(total + 1) * sizeof(WideNode));
     if (rc) return rc;
-    for (size_t i = 0; i < levels.size(); ++i) {
-        const Level &L = levels[i];
-        const uint32_t child = i + 1 < levels.size() ? levels[i + 1].off : 0u;
-        hipLaunchKernelGGL(k_wide_build, dim3(((1u << L.level) + 255) / 256), dim3(256), 0, nullptr, v.nodes,
-                           s->tris.as<TriRec>(), v.shade, s->wide.as<WideNode>(), L.off, L.level, L.step, child,
-                           v.wide_lo[0], v.wide_lo[1], v.wide_lo[2], scale);
+    uint32_t *found = reinterpret_cast<uint32_t *>(s->wide.as<WideNode>() + total), got = 0;
+    while (true) {
+        RM_HIP(hipMemset(found, 0, sizeof(WideNode)));
+        for (size_t i = levels.size(); i-- > 0;) {  // children first: their E
+            const Level &L = levels[i];
+            const uint32_t child = i + 1 < levels.size() ? levels[i + 1].off : 0u;
+            hipLaunchKernelGGL(k_wide_build, dim3(((1u << L.level) + 255) / 256), dim3(256), 0, nullptr, v.nodes,
+                               s->tris.as<TriRec>(), v.shade, s->wide.as<WideNode>(), L.off, L.level, L.step, child,
+                               v.wide_lo[0], v.wide_lo[1], v.wide_lo[2], scale, reach, big, found);
+        }
+        RM_HIP(hipGetLastError());
+        // waits: the caller may use the scene on any stream next
+        RM_HIP(hipMemcpy(&got, found, sizeof(got), hipMemcpyDeviceToHost));
+        if (got <= MAX_BIG) break;
+        big = INFINITY;  // too many: the tree bounds them all
     }
-    RM_HIP(hipGetLastError());
-    // the caller may use the scene on any stream next
-    RM_HIP(hipStreamSynchronize(nullptr));
+    v.n_big = (int32_t)got;
+    v.big = found + 1;
     v.wide = s->wide.as<WideNode>();
     return RM_OK;
 }

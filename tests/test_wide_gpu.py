@@ -38,6 +38,14 @@ def walls(n):
     return np.ascontiguousarray(np.stack(out), dtype=np.float32)
 
 
+def needles(n):
+    """Triangles whose first edge's square is below the float range."""
+    v = soup(n, 18, 0.6)
+    v[:, 0] = 0.0
+    v[:, 1] = np.float32([1e-20, 1e-21, 0.0])
+    return v
+
+
 SCENES = {
     "one_leaf": lambda: soup(10, 1, 0.5), "two_leaves": lambda: soup(11, 2, 0.5), "soup20": lambda: soup(20, 3, 0.4),
     "soup21": lambda: soup(21, 4, 0.4), "soup48": lambda: soup(48, 5, 0.3), "soup49": lambda: soup(49, 6, 0.3),
@@ -45,6 +53,8 @@ SCENES = {
     "slivers": lambda: (soup(60, 15, 0.8) * np.array([1, 1e-4, 1]) + np.array([90, 40, -7])).astype(np.float32),
     "soup80": lambda: soup(80, 7, 0.3), "soup81": lambda: soup(81, 8, 0.3), "soup1301": lambda: soup(1301, 9),
     "soup7001": lambda: soup(7001, 10, 0.05), "walls": lambda: walls(9),
+    "needles3": lambda: np.concatenate([soup(900, 16, 0.2), needles(3)]),
+    "needles12": lambda: np.concatenate([soup(900, 17, 0.2), needles(12)]),
     "doubled": lambda: np.repeat(soup(700, 11, 0.2), 2, axis=0),
     "ground": lambda: np.concatenate([soup(3000, 12, 0.02) * np.float32(0.2),
                                       np.array([[[-40, 0, -40], [40, 0, -40], [40, 0, 40]],
@@ -108,6 +118,70 @@ def test_bit_exact(dev, scene):
         aim = aim.astype(np.float32)
         occ = S.trace_any(rd, aim_dev=torch.from_numpy(aim).to(dev))
         assert np.array_equal(occ.cpu().numpy(), OS.any(r, aims=aim)), (scene, kind)
+
+
+def mixed(n, n_big, ext, small, big, seed):
+    """n triangles over ext units, n_big of them large and tilted."""
+    r = np.random.default_rng(seed)
+    c = r.random((n, 1, 3)) * ext
+    v = c + small * np.exp(r.normal(0, 0.7, (n, 1, 1))) * (r.random((n, 3, 3)) - 0.5)
+    i = r.permutation(n)[:n_big]
+    v[i] = c[i] + big * (r.random((n_big, 3, 3)) - 0.5)
+    return v.astype(np.float32), i
+
+
+def grazing(v, idx, n, length, dev, seed):
+    """Rays nearly in the plane of a large triangle, n.d between 0.8e-4 and
+    1.6e-3 |e1| (tests reject below 1e-4 |e1|), aimed at points in it and a
+    little outside: computed t, u and v are least accurate there."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(seed)
+    rnd = lambda *s: torch.rand(*s, generator=g, device=dev, dtype=torch.float64)  # noqa: E731
+    T = torch.tensor(v[idx], device=dev, dtype=torch.float64)[torch.randint(0, len(idx), (n,), generator=g, device=dev)]
+    e1, e2 = T[:, 1] - T[:, 0], T[:, 2] - T[:, 0]
+    m = torch.cross(e1, e2, dim=1)
+    l, l1 = m.norm(dim=1, keepdim=True), e1.norm(dim=1, keepdim=True)
+    x, a = e1 / l1, rnd(n, 1) * 6.2832
+    k = 0.8e-4 * 20.0 ** rnd(n, 1) * l1 / l
+    d = length * (x * torch.cos(a) + torch.cross(m / l, x, dim=1) * torch.sin(a)) + m / l * torch.where(rnd(n, 1) < 0.5, -k, k)
+    b = rnd(n, 2)
+    b = torch.where(b.sum(1, keepdim=True) > 1, 1 - b, b) * 1.1 - 0.05
+    o = T[:, 0] + b[:, :1] * e1 + b[:, 1:] * e2 - d / d.norm(dim=1, keepdim=True) * rnd(n, 1) * float(np.ptp(v))
+    return torch.cat([o, d], 1).float().contiguous()
+
+
+# small and large scenes, some in and some outside the tree's range of sizes,
+# and long directions, whose computed distances err as in a larger scene
+@pytest.mark.parametrize("n, n_big, ext, small, big", [
+    (200, 20, 20, 1, 8), (200, 20, 300, 20, 200), (200, 200, 25, 15, 15), (2000, 50, 25, 0.5, 15), (2000, 50, 100, 2, 70),
+    (2000, 50, 1000, 20, 700), (2000, 4, 25, 0.5, 20), (50000, 100, 10, 0.05, 5)])
+def test_grazing(dev, n, n_big, ext, small, big):
+    """Rays for which a triangle's computed t can lie before its own box."""
+    for seed in range(3):
+        v, idx = mixed(n, n_big, ext, small, big, seed)
+        k = len(v)
+        m = rm._lib.RmMaterial(roughness=0.8, opacity=1.0, ior=1.0, albedo_tex=-1, normal_tex=-1, emissive_tex=-1, specular_tex=-1)
+        desc, keep = make_desc(v, np.zeros((k, 3, 2)), np.zeros(k), np.zeros(k), [m], [])
+        S, OS = rm.Scene(desc), O.OracleScene(desc)
+        for length in (1.0, 10.0, 60.0, 400.0):
+            r = grazing(v, idx, 1 << 20, length, dev, seed)
+            aim = 0.5 * ext / length
+            t, ids = S.trace_closest(r)
+            occ = S.trace_any(r, aim=aim)
+            try:
+                rm.set_tuning(rm.TUNE_TRACE_VARIANT, 0)
+                t0, i0 = S.trace_closest(r)
+                occ0 = S.trace_any(r, aim=aim)
+                torch.cuda.synchronize()
+            finally:
+                rm.set_tuning(rm.TUNE_TRACE_VARIANT, 3)
+            bad = (ids != i0) | (t.view(torch.int32) != t0.view(torch.int32)) | (occ != occ0)
+            assert not bool(bad.any()), (seed, length, int(bad.sum()))
+            # the walk compared with, against the oracle
+            few = r[:2000].cpu().numpy()
+            to, io = OS.closest(few)
+            assert np.array_equal(i0[:2000].cpu().numpy(), io)
+            assert np.array_equal(t0[:2000].cpu().numpy().view(np.uint32), to.view(np.uint32))
 
 
 @pytest.mark.parametrize("tris", [36, 3001])
