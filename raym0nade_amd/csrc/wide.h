@@ -7,17 +7,18 @@
 // running t_max), the reference visits a leaf for certain when G holds and L
 // lies below its running t_max: the boxes of the leaf's ancestors contain the
 // leaf's, and every operation of the slab test is monotone, so theirs pass
-// too.  Let a walk end with closest hit t* in one leaf, t2 being the least t
-// it accepted in other leaves, and let no triangle that it did not test have a
+// too.  Let a walk end with closest hit t* in one leaf, t2 being the next t
+// that it accepted, and let no triangle that it did not test have a
 // computed t below lim(t*), somewhat more than t*.  Then
 //     G(leaf)  and  t* < t2  and  L(leaf) < min(t2, lim(t*))
 // proves that the reference ends with the same triangle: its t_max stays
 // >= min(t2, lim(t*)) until it reaches that leaf, and > t* then, and later
-// hits are no closer.  The walk here tests a superset of the
+// hits are no closer.  Where a triangle of one other leaf has the same t
+// (doubled triangles), first_of says which leaf comes first.  The walk here tests a superset of the
 // reference's boxes with cheap arithmetic (fused multiply-adds on 16-bit
 // boxes, rounded outward, with margins that cover every rounding) and checks
 // this certificate once per ray, on the reference's own box.  Where it fails
-// -- two hits within a rounding error of each other -- the ray is walked
+// -- hits of different leaves within a rounding error of each other -- the ray is walked
 // again in the reference's order, by the same lane (RefWalker).  A shadow ray
 // is blocked for certain when an accepted t < aim lies in a leaf with G and
 // L < aim.
@@ -169,10 +170,13 @@ __device__ __forceinline__ bool wide_ray(const SceneView &S, V3 o, V3 d, float t
     return ok;
 }
 
+// The number of a triangle's leaf in the implicit heap.
+__device__ __forceinline__ uint32_t leaf_of(const TriRec *tris, int32_t slot) { return __float_as_uint(tris[slot].e2[3]); }
+
 // G(leaf) and L(leaf) < limit for the leaf that holds triangle `slot`.
 __device__ __forceinline__ bool leaf_certain(const PairNode *nodes, const TriRec *tris, int32_t slot, V3 o, V3 d,
                                              float tmin, float limit) {
-    const uint32_t c = __float_as_uint(tris[slot].e2[3]);  // the leaf's number in the implicit heap
+    const uint32_t c = leaf_of(tris, slot);
     const float4 *P = reinterpret_cast<const float4 *>(nodes + (c >> 1));
     const float4 A = P[0], B = P[1], C = P[2];
     float tL = tmin, tR = INFINITY;
@@ -181,6 +185,25 @@ __device__ __forceinline__ bool leaf_certain(const PairNode *nodes, const TriRec
     else
         box_test(ray_pre(o, d), A.x, A.y, A.z, A.w, B.x, B.y, tL, tR);
     return tL < tR && tL < limit;
+}
+
+// Of two triangles of different leaves, the one whose leaf the reference comes
+// to first if it visits both: it enters first the child of their leaves'
+// common ancestor whose box the ray enters first, child 1 of equal ones.
+__device__ __forceinline__ int32_t first_of(const PairNode *nodes, const TriRec *tris, int32_t x, int32_t y, V3 o, V3 d,
+                                            float tmin) {
+    uint32_t a = leaf_of(tris, x), b = leaf_of(tris, y);
+    const int up = (int)__clz(a) - (int)__clz(b);
+    a >>= up < 0 ? -up : 0;
+    b >>= up > 0 ? up : 0;
+    const int k = 32 - (int)__clz(a ^ b);
+    const float4 *P = reinterpret_cast<const float4 *>(nodes + (a >> k));
+    const float4 A = P[0], B = P[1], C = P[2];
+    const RayPre r = ray_pre(o, d);
+    float tL0 = tmin, tR0 = INFINITY, tL1 = tmin, tR1 = INFINITY;
+    box_test(r, A.x, A.y, A.z, A.w, B.x, B.y, tL0, tR0);
+    box_test(r, B.z, B.w, C.x, C.y, C.z, C.w, tL1, tR1);
+    return ((a >> (k - 1)) & 1u) == (tL0 < tL1 ? 0u : 1u) ? x : y;
 }
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -356,35 +379,60 @@ struct WideWalker {
         next(lim);
     }
 
-    // Tests a triangle (twice is as good as once).
-    __device__ __forceinline__ void test(const TriRec *tris, uint32_t i, V3 o, V3 d, float tmin) {
+    // Tests a triangle (twice is as good as once).  Of equal t in one leaf the
+    // first triangle stands, as in the reference; an equal t of another leaf
+    // is kept in tie, or -1 there for two such leaves.  tie is memory, touched
+    // only then: another register would cost every walk 4%.
+    __device__ __forceinline__ void test(const TriRec *tris, uint32_t i, V3 o, V3 d, float tmin, volatile int32_t &tie) {
         TriRec T = load_tri(tris, i);
         // the whole record at once: v0 loaded past the first rejection
         // would cost a second memory latency
         asm volatile("" : "+v"(T.p[0]), "+v"(T.p[1]), "+v"(T.p[2]));
         const float t = tri_test_flat(o, d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
                                       V3{T.e2[0], T.e2[1], T.e2[2]});
-        if (tmin < t && t < t2) {
+        if (tmin < t && t <= t2) {
             if (t < tmax) {
                 t2 = tmax;
                 tmax = t;
                 best = (int32_t)i;
-            } else if (best != (int32_t)i) {
+            } else if (t > tmax) {
                 t2 = t;
+            } else if (best >= 0 && best != (int32_t)i) {
+                const uint32_t leaf = leaf_of(tris, (int32_t)i);
+                const int32_t was = t2 > tmax ? -1 : tie;
+                if (leaf == leaf_of(tris, best)) {
+                    best = min(best, (int32_t)i);
+                } else if (t2 > tmax) {
+                    tie = (int32_t)i;
+                    t2 = tmax;
+                } else {
+                    tie = was >= 0 && leaf == leaf_of(tris, was) ? min(was, (int32_t)i) : -1;
+                }
             }
         }
     }
+    // After the walk (of the tree: only its tests write tie): with t2 == tmax,
+    // tie is the one other leaf's triangle with that t, or -1.  Every other is
+    // beyond it, so the least t2 that says so will do.
+    __device__ __forceinline__ void settle(const SceneView &S, V3 o, V3 d, float tmin, const volatile int32_t &tie) {
+        if (best < 0 || t2 != tmax) return;
+        const int32_t other = tie;
+        if (other >= 0) {
+            best = first_of(S.nodes, S.tris, best, other, o, d, tmin);
+            t2 = __uint_as_float(__float_as_uint(tmax) + 1u);
+        }
+    }
     // Those that the boxes' growth leaves out.
-    __device__ __forceinline__ void test_big(const SceneView &S, V3 o, V3 d, float tmin) {
-        for (int k = 0; k < S.n_big; ++k) test(S.tris, S.big[k], o, d, tmin);
+    __device__ __forceinline__ void test_big(const SceneView &S, V3 o, V3 d, float tmin, volatile int32_t &tie) {
+        for (int k = 0; k < S.n_big; ++k) test(S.tris, S.big[k], o, d, tmin, tie);
     }
 
     // Tests the first run of l.
-    __device__ __forceinline__ void step_run(const TriRec *tris, const WideRay &r, float tmin) {
+    __device__ __forceinline__ void step_run(const TriRec *tris, const WideRay &r, float tmin, volatile int32_t &tie) {
         const uint32_t first = (lx >> 6) & 0x1ffffffu, c = (lx >> 2) & 15u, k = ly & 3u;
         const uint32_t end = first + (c * (k + 1u) >> 2);
         for (uint32_t i = first + (c * k >> 2); i < end; ++i) {
-            test(tris, i, r.o, r.d, tmin);
+            test(tris, i, r.o, r.d, tmin, tie);
         }
         drop_first(ly);
         const float lim = wide_limit(tmax);
@@ -400,6 +448,8 @@ struct RefWalker {
     int sp;
     uint32_t cur;
 
+    // the wide walk's tie, while this one is not under way
+    __device__ __forceinline__ volatile int32_t &tie() { return *reinterpret_cast<volatile int32_t *>(&e[0].x); }
     __device__ __forceinline__ void init(uint32_t root_leaf) {
         sp = 0;
         cur = root_leaf ? root_leaf | 0x80000000u : 1u;
@@ -508,6 +558,8 @@ __device__ __forceinline__ void flat_tris(const SceneView &S, V3 o, V3 d, float 
         }
         pending &= ~__ballot(mine);
     }
+    int32_t tie = -1;                    // a triangle of another leaf with best's t
+    uint32_t leaf = 0u, tie_leaf = 0u;   // best's and tie's
     while (mask[0] | mask[1]) {
         uint32_t i;
         if (mask[0]) {
@@ -520,12 +572,18 @@ __device__ __forceinline__ void flat_tris(const SceneView &S, V3 o, V3 d, float 
         const TriRec T = load_tri(S.tris, i);
         const float t = tri_test_flat(o, d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
                                       V3{T.e2[0], T.e2[1], T.e2[2]});
-        const bool in = tmin < t && t < t2, first = t < tmax;
-        t2 = in ? (first ? tmax : t) : t2;
+        const uint32_t l = __float_as_uint(T.e2[3]);
+        const bool in = tmin < t && t < t2, first = t < tmax, other = l != leaf;
+        const bool tied = in && other && t == tmax && (tie < 0 || l == tie_leaf);
+        t2 = in && (first ? other || tie >= 0 : other && !tied) ? (first ? tmax : t) : t2;
+        tie = in && first ? -1 : tied && tie < 0 ? (int32_t)i : tie;
+        tie_leaf = tied ? l : tie_leaf;
+        leaf = in && first ? l : leaf;
         best = in && first ? (int32_t)i : best;
         tmax = in && first ? t : tmax;
         if (ANY && tmax < aim) break;
     }
+    if (tie >= 0) best = first_of(S.nodes, S.tris, best, tie, o, d, tmin);
 }
 
 // Whether the result of flat_tris or of a finished wide walk stands.
@@ -543,16 +601,17 @@ template <bool ANY, bool LDSW>
 __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, float tmin, float &tmax, float aim) {
     WideWalker<typename std::conditional<LDSW, WideLds, WidePrivate>::type> w;
     WideRay r;
+    RefWalker ref;
     w.stk.bind();
     w.init(tmax);
     bool sure = true;
     if (S.flat) {
         flat_tris<ANY>(S, o, d, tmin, aim, w.tmax, w.t2, w.best);
     } else if (S.wide && wide_ray(S, o, d, tmin, r)) {
-        w.test_big(S, o, d, tmin);
+        w.test_big(S, o, d, tmin, ref.tie());
         while (!(ANY && w.tmax < aim)) {
             if (w.has_run()) {
-                w.step_run(S.tris, r, tmin);
+                w.step_run(S.tris, r, tmin, ref.tie());
                 if (ANY && w.tmax < aim) break;
             } else if (w.has_node()) {
                 w.step_node(S.wide, S.wide_scale, r, tmin);
@@ -560,11 +619,11 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
                 break;
             }
         }
+        w.settle(S, o, d, tmin, ref.tie());
     } else {
         sure = false;
     }
     if (!sure || !hit_sure<ANY>(S, o, d, tmin, aim, w.tmax, w.t2, w.best)) {
-        RefWalker ref;
         ref.init((uint32_t)S.root_leaf);
         w.tmax = tmax;
         w.best = -1;
@@ -636,6 +695,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
             // results of the lanes that finished
             if (ray != WIDE_NONE && !walking) {
                 const SceneView &S = src.scene();
+                if (!S.flat) w.settle(S, r.o, r.d, tmin, ref.tie());  // (flat_tris has its own)
                 if (hit_sure<ANY>(S, r.o, r.d, tmin, aim, w.tmax, w.t2, w.best)) {
                     src.store(ray, w.tmax, w.best, aim);
                     ray = WIDE_NONE;
@@ -675,7 +735,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
                         ref.init((uint32_t)S.root_leaf);
                         w.stop();
                     } else {
-                        w.test_big(S, o, d, tmin);
+                        w.test_big(S, o, d, tmin, ref.tie());
                         if (ANY && w.tmax < aim) w.stop();
                     }
                 }
@@ -696,7 +756,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
         const uint32_t nr = (uint32_t)__popcll(runs), nw = (uint32_t)__popcll(nodes | runs);
         if (nr && (!nodes || 64u * nr >= (uint32_t)phases * nw)) {
             if (w.has_run()) {
-                w.step_run(src.scene().tris, r, tmin);
+                w.step_run(src.scene().tris, r, tmin, ref.tie());
                 if (ANY && w.tmax < aim) w.stop();
             }
         } else if (w.has_node()) {

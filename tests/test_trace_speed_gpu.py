@@ -1,0 +1,79 @@
+"""Calls for which the default walk has a slow way out: timed against the walk
+of the binary tree (trace variant 3, four triangles a step) at the settings
+that suit it, which the default has to come near at least."""
+import contextlib
+
+import numpy as np
+import pytest
+import torch
+
+import raym0nade_amd as rm
+from cutout_util import make_desc
+
+pytestmark = pytest.mark.gpu
+
+BINARY = {rm.TUNE_TRIS_PER_STEP: 4, rm.TUNE_FETCH_MIN: 48}
+
+
+@contextlib.contextmanager
+def tuned(values):
+    old = {k: rm.get_tuning(k) for k in values}
+    try:
+        for k, v in values.items():
+            rm.set_tuning(k, v)
+        yield
+    finally:
+        for k, v in old.items():
+            rm.set_tuning(k, v)
+
+
+def ms(fn, reps=5):
+    """The least of a few runs, after one to warm up."""
+    fn()
+    best = float("inf")
+    for _ in range(reps):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        fn()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b))
+    return best
+
+
+def both(scene, rays, **kw):
+    t = torch.empty(rays.shape[0], device=rays.device)
+    i = torch.empty(rays.shape[0], device=rays.device, dtype=torch.int32)
+    run = lambda: scene.trace_closest(rays, t_out=t, id_out=i, **kw)  # noqa: E731
+    own = ms(run)
+    with tuned(BINARY):
+        return own, ms(run)
+
+
+def make(v):
+    v = np.ascontiguousarray(v, np.float32)
+    m = rm._lib.RmMaterial(roughness=0.8, opacity=1.0, ior=1.0, albedo_tex=-1, normal_tex=-1, emissive_tex=-1, specular_tex=-1)
+    k = len(v)
+    desc, keep = make_desc(v, np.zeros((k, 3, 2)), np.zeros(k), np.zeros(k), [m], [])
+    S = rm.Scene(desc)
+    S.arrays = keep
+    return S
+
+
+def soup(n, seed, size):
+    r = np.random.default_rng(seed)
+    return (r.random((n, 1, 3)) + size * (r.random((n, 3, 3)) - 0.5)).astype(np.float32)
+
+
+def uniform(n, dev, length=1.0):
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    d = torch.randn(n, 3, generator=g, device=dev)
+    return torch.cat([torch.rand(n, 3, generator=g, device=dev), d / d.norm(dim=1, keepdim=True) * length], 1).contiguous()
+
+
+def test_doubled_triangles(dev):
+    """Every hit is one of two at the same distance, some in different leaves."""
+    v = soup(100000, 1, 0.015)
+    own, binary = both(make(np.concatenate([v, v])), uniform(1 << 20, dev))
+    assert own < 1.2 * binary, (own, binary)

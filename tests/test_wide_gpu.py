@@ -56,6 +56,8 @@ SCENES = {
     "needles3": lambda: np.concatenate([soup(900, 16, 0.2), needles(3)]),
     "needles12": lambda: np.concatenate([soup(900, 17, 0.2), needles(12)]),
     "doubled": lambda: np.repeat(soup(700, 11, 0.2), 2, axis=0),
+    "twice": lambda: np.concatenate([soup(701, 11, 0.2)] * 2), "thrice": lambda: np.concatenate([soup(501, 11, 0.2)] * 3),
+    "twice_flat": lambda: np.concatenate([soup(31, 11, 0.4)] * 2), "thrice_flat": lambda: np.concatenate([soup(21, 11, 0.4)] * 3),
     "ground": lambda: np.concatenate([soup(3000, 12, 0.02) * np.float32(0.2),
                                       np.array([[[-40, 0, -40], [40, 0, -40], [40, 0, 40]],
                                                 [[-40, 0, -40], [40, 0, 40], [-40, 0, 40]]], np.float32)]),
