@@ -478,7 +478,8 @@ enum rm_tune_key {
                                            tree; 1 and 4 (a one-ray step walk and two walks per lane) are
                                            retired and rejected */
     RM_TUNE_PERSISTENT_BLOCKS_PER_CU = 1, /* resident 256-lane blocks per CU for variants 2, 3 (default 8) */
-    RM_TUNE_FETCH_MIN = 2,              /* idle lanes before a wave claims new rays (default 16) */
+    RM_TUNE_FETCH_MIN = 2,              /* idle lanes before a wave claims new rays (default 16; the walk
+                                           of the binary tree takes 48 for it) */
     RM_TUNE_RAY_SORT = 3,               /* ray reordering for trace calls: 0 never, 1 when consecutive
                                            origins are far apart, 2 always, 3 as 1 with a radix sort
                                            of the bins (rocPRIM) instead of the counting sort, 4 as 3

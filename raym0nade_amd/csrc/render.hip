@@ -1993,7 +1993,7 @@ static int32_t render_jobs(const std::vector<HostJob> &hj_in, DevBuf &work, hipS
     if (graph) RM_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     const int mw = tuning().render_min_waves;  // 1, 3 or 4
     const unsigned gpers = (unsigned)(device_cu_count() * tuning().persistent_blocks_per_cu);
-    const int fetch_min = tuning().fetch_min;
+    const int fetch_min = fetch_lanes(tuning(), wide);
     const int phases = tuning().walk_phases;
     auto shadow = counting ? (lds_walk ? (tps == 1 ? k_shadow<true, 1, true> : tps == 2 ? k_shadow<true, 2, true>
                                           : tps == 4 ? k_shadow<true, 4, true> : k_shadow<true, 0, true>)

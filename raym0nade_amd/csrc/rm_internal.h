@@ -132,7 +132,7 @@ struct Tuning {
     int trace_variant = 3;        // 0 stack walk, 2 persistent step walk, 3 same with LDS stacks, or with
                                   // tris_per_step 0 the four-wide walk (wide.h)
     int persistent_blocks_per_cu = 8;
-    int fetch_min = 16;           // idle lanes before a wave claims new rays
+    int fetch_min = 16;           // idle lanes before a wave claims new rays (fetch_lanes)
     int ray_sort = 5;             // 0 never, 1 when consecutive origins are far apart, 2 always,
                                   // 3 as 1 with a radix sort (rocPRIM) instead of the counting sort,
                                   // 4 as 3 with the library's own radix sort (skipped on the device
@@ -152,6 +152,13 @@ struct Tuning {
 Tuning &tuning();
 // Whether walks are the four-wide one by default (variant 3, whole leaves).
 inline bool wide_chosen(const Tuning &t) { return t.trace_variant == 3 && t.tris_per_step == 0; }
+// Idle lanes before a wave claims new rays: the default, 16, is the four-wide
+// walk's best; the binary tree's walk then takes its own, 48 (1M uniform rays
+// among 500 triangles: 552 us, with 16 idle lanes 798).
+constexpr int FETCH_DEFAULT = 16, FETCH_BINARY = 48;
+inline int fetch_lanes(const Tuning &t, bool wide) {
+    return !wide && t.fetch_min == FETCH_DEFAULT ? FETCH_BINARY : t.fetch_min;
+}
 int device_cu_count();
 
 }  // namespace rm

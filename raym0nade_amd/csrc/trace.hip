@@ -892,6 +892,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, next);
         const int nl = std::min(std::max(1, (int)s->view.depth), T.lds_stack_entries);
         const bool util = T.trace_util != 0 && !fixed;
+        const int fetch = fetch_lanes(T, wide);
         if (wide) {
             // every wave a few rays, or the whole machine
             const uint32_t most = (uint32_t)device_cu_count() * T.persistent_blocks_per_cu * (TRACE_BLOCK / 64);
@@ -900,7 +901,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
             pgrid = (waves + TRACE_BLOCK / 64 - 1) / (TRACE_BLOCK / 64);
             hipLaunchKernelGGL(k_trace_wide<ANY>, dim3(pgrid), dim3(TRACE_BLOCK), wide_lds_bytes(s->view.depth), st,
                                s->view, rays, (uint32_t)n, tmin, t0, aim_dev, t_out, id_out, occ, next, per,
-                               T.fetch_min, (const uint32_t *)order, (const int *)flag, T.walk_phases);
+                               fetch, (const uint32_t *)order, (const int *)flag, T.walk_phases);
         } else if (T.trace_variant == 3) {
             unsigned long long *ud = nullptr;
             if (util) {
@@ -919,11 +920,11 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
                                 : T.tris_per_step == 4 ? k_trace_persistent<ANY, true, 4>
                                                        : k_trace_persistent<ANY, true, 0>);
             hipLaunchKernelGGL(kern, dim3(pgrid), dim3(TRACE_BLOCK), (size_t)nl * TRACE_BLOCK * 8, st, s->view, rays, n,
-                               tmin, t0, aim_dev, t_out, id_out, occ, next, T.fetch_min, (const uint32_t *)order,
+                               tmin, t0, aim_dev, t_out, id_out, occ, next, fetch, (const uint32_t *)order,
                                (const int *)flag, nl, ud, T.walk_phases);
         } else
             hipLaunchKernelGGL((k_trace_persistent<ANY, false, 0>), dim3(pgrid), dim3(TRACE_BLOCK), 0, st, s->view, rays,
-                               n, tmin, t0, aim_dev, t_out, id_out, occ, next, T.fetch_min, (const uint32_t *)order,
+                               n, tmin, t0, aim_dev, t_out, id_out, occ, next, fetch, (const uint32_t *)order,
                                (const int *)flag, 0);
     } else if (ANY) {
         hipLaunchKernelGGL(k_trace_any<0>, dim3(grid), dim3(TRACE_BLOCK), 0, st, s->view, rays, n, tmin, t0, aim_dev, occ,

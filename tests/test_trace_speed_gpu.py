@@ -41,12 +41,12 @@ def ms(fn, reps=5):
     return best
 
 
-def both(scene, rays, **kw):
+def both(scene, rays, binary=BINARY, **kw):
     t = torch.empty(rays.shape[0], device=rays.device)
     i = torch.empty(rays.shape[0], device=rays.device, dtype=torch.int32)
     run = lambda: scene.trace_closest(rays, t_out=t, id_out=i, **kw)  # noqa: E731
     own = ms(run)
-    with tuned(BINARY):
+    with tuned(binary):
         return own, ms(run)
 
 
@@ -77,3 +77,12 @@ def test_doubled_triangles(dev):
     v = soup(100000, 1, 0.015)
     own, binary = both(make(np.concatenate([v, v])), uniform(1 << 20, dev))
     assert own < 1.2 * binary, (own, binary)
+
+
+def test_scene_outside_the_trees_range(dev):
+    """Far from the origin the binary tree is walked, at its own claim threshold."""
+    S = make(soup(500, 2, 0.2) + np.float32(2e4))
+    r = uniform(1 << 20, dev)
+    r[:, :3] += 2e4
+    own, binary = both(S, r.contiguous(), {rm.TUNE_FETCH_MIN: 48})
+    assert own < 1.15 * binary, (own, binary)
