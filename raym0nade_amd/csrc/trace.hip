@@ -770,7 +770,9 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
     char *ws = nullptr;
     std::unique_lock<std::mutex> ws_lock;
     // The wide walk is sorted less: only large incoherent batches gain.
-    const bool wide = wide_chosen(T) && (s->view.wide || s->view.flat) && !(T.trace_util && !fixed) &&
+    // (With a negative tmin every ray of it would walk in the reference's
+    // order, which the binary walk's kernels do faster.)
+    const bool wide = wide_chosen(T) && (s->view.flat || (s->view.wide && tmin >= 0.0f)) && !(T.trace_util && !fixed) &&
                       n < (int64_t)0xf0000000;
     const int64_t sort_min = !wide ? 4096 : s->view.n_tris < WIDE_SORT_TRIS ? INT64_MAX : ANY ? 2 * WIDE_SORT_RAYS : WIDE_SORT_RAYS;
     if ((T.ray_sort == 4 || T.ray_sort == 5) && n >= sort_min) {

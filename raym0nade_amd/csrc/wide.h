@@ -104,6 +104,13 @@ struct WideRay {
     float inv[3];
     float nr[3], fr[3];
     float err;       // WIDE_ERR |d| / scale: a box grows by err E distance; negative for a ray with parallel axes
+
+    // For RefWalker, which needs the wide tree's values no more.
+    __device__ __forceinline__ void reciprocals(V3 dir) {
+        inv[0] = 1.0f / dir.x;
+        inv[1] = 1.0f / dir.y;
+        inv[2] = 1.0f / dir.z;
+    }
 };
 
 // How far from a triangle the test accepts a ray: with the computed a, u, v
@@ -127,8 +134,9 @@ struct WideRay {
 // |e2| over the size of a scene for |d| = 1: over 10 / 30 / 100 units, closest
 // hits among a million triangles take 0.57 / 0.73 / 1.33 of the binary walk's
 // time, 5000 take 0.65 / 0.88 / 1.75, 300 take 0.70 / 1.04 / 1.64.  WIDE_FAR bounds it for a
-// ray, which RefWalker serves otherwise, more slowly than the binary walk's
-// kernels: at 1.3 the grown boxes take 1.1 to 1.9 of those kernels' time.
+// ray over its distance from the scene's middle, or half the scene's size;
+// RefWalker serves others.  Among spheres over 8 units that bound is 1.0 for
+// |d| = 20: @F; over 240 units, from outside, 3: 4 to 6 times, with RefWalker 1.3.
 constexpr float WIDE_ERR = 0.0126f;
 constexpr float WIDE_SCENE = 0.4f, WIDE_FAR = 1.5f;
 // The entry distances' slack below the running t_max: 3 eps_zero of rayInBox,
@@ -151,7 +159,7 @@ __device__ __forceinline__ bool wide_ray(const SceneView &S, V3 o, V3 d, float t
     const float sum = ((p[0] + p[1]) + p[2]) + ((d.x + d.y) + d.z);
     r.err = length(d) * S.wide_rscale * WIDE_ERR;
     const bool ok = tmin >= 0.0f && far < 4e6f && dmax > 1e-3f && dmax < 1e9f && sum == sum &&
-                    r.err * (off + S.wide_reach) < WIDE_FAR;
+                    r.err * fmaxf(off, 0.5f * S.wide_reach) < WIDE_FAR;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const bool par = fabsf(dv[k]) < T_EPS;
@@ -454,9 +462,9 @@ struct RefWalker {
         sp = 0;
         cur = root_leaf ? root_leaf | 0x80000000u : 1u;
     }
-    // True when the walk has finished (or tmax < aim).
-    __device__ __forceinline__ bool step(const PairNode *bin, const TriRec *tris, V3 o, V3 d, float tmin, float aim,
-                                         float &tmax, int32_t &best) {
+    // True when the walk has finished (or tmax < aim).  inv: 1 / d.
+    __device__ __forceinline__ bool step(const PairNode *bin, const TriRec *tris, V3 o, V3 d, const float (&inv)[3], float tmin,
+                                         float aim, float &tmax, int32_t &best) {
         if (cur & 0x80000000u) {
             const uint32_t first = (cur & 0x7fffffffu) >> LEAF_SHIFT, cnt = cur & LEAF_MASK;
             for (uint32_t i = first; i < first + cnt; ++i) {
@@ -472,10 +480,15 @@ struct RefWalker {
             const float4 *P = reinterpret_cast<const float4 *>(bin + cur);
             const float4 A = P[0], B = P[1], C = P[2];
             const uint2 L = *reinterpret_cast<const uint2 *>(&P[3]);
-            const RayPre r = ray_pre(o, d);
+            const RayPre r{o, d, {inv[0], inv[1], inv[2]}, {fabsf(d.x) < T_EPS, fabsf(d.y) < T_EPS, fabsf(d.z) < T_EPS}};
             float tL0 = tmin, tR0 = tmax, tL1 = tmin, tR1 = tmax;
-            box_test(r, A.x, A.y, A.z, A.w, B.x, B.y, tL0, tR0);
-            box_test(r, B.z, B.w, C.x, C.y, C.z, C.w, tL1, tR1);
+            if (r.par[0] || r.par[1] || r.par[2]) {
+                box_test(r, A.x, A.y, A.z, A.w, B.x, B.y, tL0, tR0);
+                box_test(r, B.z, B.w, C.x, C.y, C.z, C.w, tL1, tR1);
+            } else {
+                box_test_fast(r, A.x, A.y, A.z, A.w, B.x, B.y, tL0, tR0);
+                box_test_fast(r, B.z, B.w, C.x, C.y, C.z, C.w, tL1, tR1);
+            }
             const uint32_t ref0 = L.x ? (L.x | 0x80000000u) : (cur << 1);
             const uint32_t ref1 = L.y ? (L.y | 0x80000000u) : (cur << 1 | 1u);
             const bool f0 = tL0 < tL1;
@@ -625,9 +638,10 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
     }
     if (!sure || !hit_sure<ANY>(S, o, d, tmin, aim, w.tmax, w.t2, w.best)) {
         ref.init((uint32_t)S.root_leaf);
+        r.reciprocals(d);
         w.tmax = tmax;
         w.best = -1;
-        while (!ref.step(S.nodes, S.tris, o, d, tmin, aim, w.tmax, w.best)) {
+        while (!ref.step(S.nodes, S.tris, o, d, r.inv, tmin, aim, w.tmax, w.best)) {
         }
     }
     tmax = w.tmax;
@@ -702,6 +716,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
                 } else {
                     in_ref = true;
                     ref.init((uint32_t)S.root_leaf);
+                    r.reciprocals(r.d);
                     w.tmax = tmax0;
                     w.best = -1;
                 }
@@ -733,6 +748,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
                     } else if (!ok) {
                         in_ref = true;
                         ref.init((uint32_t)S.root_leaf);
+                        r.reciprocals(d);
                         w.stop();
                     } else {
                         w.test_big(S, o, d, tmin, ref.tie());
@@ -743,9 +759,9 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
             if (at < end) at += (uint32_t)__popcll(idle);
         }
         if (__ballot(in_ref)) {
-            if (in_ref) {
+            if (walk_turn(ref.cur, phases, in_ref) && in_ref) {
                 const SceneView &S = src.scene();
-                if (ref.step(S.nodes, S.tris, r.o, r.d, tmin, aim, w.tmax, w.best)) {
+                if (ref.step(S.nodes, S.tris, r.o, r.d, r.inv, tmin, aim, w.tmax, w.best)) {
                     src.store(ray, w.tmax, w.best, aim);
                     ray = WIDE_NONE;
                     in_ref = false;

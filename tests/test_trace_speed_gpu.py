@@ -86,3 +86,16 @@ def test_scene_outside_the_trees_range(dev):
     r[:, :3] += 2e4
     own, binary = both(S, r.contiguous(), {rm.TUNE_FETCH_MIN: 48})
     assert own < 1.15 * binary, (own, binary)
+
+
+def test_negative_tmin(dev):
+    """Rays that start behind their origin are outside what the four-wide walk proves."""
+    own, binary = both(make(soup(5000, 3, 0.05)), uniform(1 << 20, dev), tmin=-1.0)
+    assert own < 1.3 * binary, (own, binary)
+
+
+@pytest.mark.parametrize("length", [20.0, 300.0])
+def test_long_directions(dev, length):
+    """Where boxes are grown much, and where rays leave for the reference's order."""
+    own, binary = both(make(soup(5000, 3, 0.05)), uniform(1 << 17, dev, length))
+    assert own < 1.3 * binary, (own, binary)
