@@ -136,7 +136,9 @@ struct WideRay {
 // time, 5000 take 0.65 / 0.88 / 1.75, 300 take 0.70 / 1.04 / 1.64.  WIDE_FAR bounds it for a
 // ray over its distance from the scene's middle, or half the scene's size;
 // RefWalker serves others.  Among spheres over 8 units that bound is 1.0 for
-// |d| = 20: @F; over 240 units, from outside, 3: 4 to 6 times, with RefWalker 1.3.
+// |d| = 20: 0.6 to 1.25 of the
+// binary walk's time; over 240 units, from outside, 3: 4 to 6 times, with
+// RefWalker 1.3.
 constexpr float WIDE_ERR = 0.0126f;
 constexpr float WIDE_SCENE = 0.4f, WIDE_FAR = 1.5f;
 // The entry distances' slack below the running t_max: 3 eps_zero of rayInBox,
