@@ -319,11 +319,18 @@ __device__ __forceinline__ uint32_t dir_bin(V3 d, const float *box) {
 // evenly spaced pairs) exceeds `frac` of the root box diagonal; otherwise 2
 // when `box` is given (the batch is then sorted by direction: box receives
 // the range of the sampled directions' octahedral map for dir_bin), else 0.
+// wide: for the wide walk, which gains less.  Then 2 asks for shared origins
+// (all sampled ones within `frac` of the diagonal from the first) and for
+// directions that change by more than a fiftieth of their range from ray to
+// ray, as a shuffled image's do and its rows don't; with wide 2, 1 is left out.
 __global__ __launch_bounds__(256) void k_coherence(SceneView S, const float *__restrict__ rays, int64_t n, float frac,
-                                                   int *__restrict__ flag, float *__restrict__ box = nullptr) {
-    __shared__ float part[4], lo_u[4], hi_u[4], lo_v[4], hi_v[4];
+                                                   int *__restrict__ flag, float *__restrict__ box = nullptr, int wide = 0) {
+    __shared__ float part[4], lo_u[4], hi_u[4], lo_v[4], hi_v[4], turn[4], away[4];
+    float step = 0.0f, apart = 0.0f;
     float acc = 0.0f, u0 = INFINITY, u1 = -INFINITY, v0 = INFINITY, v1 = -INFINITY;
     if (n >= 2) {
+        V3 of, df;
+        load_ray(rays, 0, of, df);
         for (int s = threadIdx.x; s < 4096; s += 256) {
             int64_t k = (int64_t)s * (n - 2) / 4095;
             V3 o0, d0, o1, d1;
@@ -334,8 +341,11 @@ __global__ __launch_bounds__(256) void k_coherence(SceneView S, const float *__r
                 float u, v;
                 oct_map(d0, u, v);
                 u0 = fminf(u0, u), u1 = fmaxf(u1, u), v0 = fminf(v0, v), v1 = fmaxf(v1, v);
+                const float su = u, sv = v;
                 oct_map(d1, u, v);
                 u0 = fminf(u0, u), u1 = fmaxf(u1, u), v0 = fminf(v0, v), v1 = fmaxf(v1, v);
+                step += fabsf(u - su) + fabsf(v - sv);
+                apart = fmaxf(apart, length(o0 - of));
             }
         }
     }
@@ -345,17 +355,19 @@ __global__ __launch_bounds__(256) void k_coherence(SceneView S, const float *__r
         u1 = fmaxf(u1, __shfl_down(u1, off, 64));
         v0 = fminf(v0, __shfl_down(v0, off, 64));
         v1 = fmaxf(v1, __shfl_down(v1, off, 64));
+        step += __shfl_down(step, off, 64);
+        apart = fmaxf(apart, __shfl_down(apart, off, 64));
     }
     if ((threadIdx.x & 63) == 0) {
         const int w = threadIdx.x >> 6;
-        part[w] = acc, lo_u[w] = u0, hi_u[w] = u1, lo_v[w] = v0, hi_v[w] = v1;
+        part[w] = acc, lo_u[w] = u0, hi_u[w] = u1, lo_v[w] = v0, hi_v[w] = v1, turn[w] = step, away[w] = apart;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         float mean = (part[0] + part[1] + part[2] + part[3]) / 4096.0f;
         V3 ext{S.hi[0] - S.lo[0], S.hi[1] - S.lo[1], S.hi[2] - S.lo[2]};
         const bool spread = n >= 2 && mean > frac * length(ext);
-        *flag = spread ? 1 : (box && n >= 2 ? 2 : 0);
+        int f = spread ? (wide == 2 ? 0 : 1) : (box && n >= 2 ? 2 : 0);
         if (box) {
             for (int w = 1; w < 4; ++w) {
                 lo_u[0] = fminf(lo_u[0], lo_u[w]), hi_u[0] = fmaxf(hi_u[0], hi_u[w]);
@@ -363,11 +375,17 @@ __global__ __launch_bounds__(256) void k_coherence(SceneView S, const float *__r
             }
             // 512 cells over the sampled range; a degenerate range gets one cell
             const float du = hi_u[0] - lo_u[0], dv = hi_v[0] - lo_v[0];
+            if (wide && f == 2) {
+                const float t = (turn[0] + turn[1] + turn[2] + turn[3]) / 4096.0f;
+                const float a = fmaxf(fmaxf(away[0], away[1]), fmaxf(away[2], away[3]));
+                if (!(t > 0.02f * (du + dv) && a <= frac * length(ext))) f = 0;
+            }
             box[0] = lo_u[0];
             box[1] = lo_v[0];
             box[2] = du > 0.0f ? 512.0f / du : 0.0f;
             box[3] = dv > 0.0f ? 512.0f / dv : 0.0f;
         }
+        *flag = f;
     }
 }
 
@@ -747,12 +765,20 @@ struct FixedWorkspace {
 };
 
 // Sort modes 4 and 5 reorder a batch for the wide walk from this many rays
-// (any hits: twice as many) and triangles on; coherent batches never.  Sorted
-// / unsorted, closest hits of uniform rays: 1M triangles, 300k rays 603 / 514
-// us, 1M 1025 / 1234, 2M 1592 / 2172, 8M 4770 / 7840; 200k triangles, 1M 750 /
-// 740, 2M 1029 / 1178; 5k triangles (all in one L2), 2M 672 / 574.  Any hits
-// among 1M triangles: 1M 707 / 700, 2M 1021 / 1107.  A camera's 8M rays sorted
-// by direction: 2788 / 2544.
+// (any hits: twice as many) and triangles on.  Sorted / unsorted, closest hits
+// of uniform rays: 1M triangles, 300k rays 603 / 514 us, 1M 1025 / 1234, 2M
+// 1592 / 2172, 8M 4770 / 7840; 200k triangles, 1M 750 / 740, 2M 1029 / 1178; 5k
+// triangles (all in one L2), 2M 672 / 574.  Any hits among 1M triangles: 1M
+// 707 / 700, 2M 1021 / 1107.
+// Mode 5's order by direction, for closest hits of one origin: a camera's rows
+// are left alone (8M rays, 1M triangles 3560 / 3023, 2M in spheres 2428 / 2440);
+// its shuffled pixels 3646 / 3973 and 2468 / 2897, with 1M rays 1019 / 1164 and
+// 599 / 658; directions from a point 4574 / 4955 and 2349 / 2391.  In small
+// scenes the probe shows, so from four times as many rays: 5k triangles, 8M
+// shuffled 2664 / 3138, 4M 1422 / 1695, 1M 539 / 570 of which 50 us the probe and
+// the kernels that it skips.  Ambient occlusion's rays (neighbouring origins,
+// any direction) lose by either order: 8M, 1M triangles, by cells 4037, by
+// direction 4067, unsorted 3824.
 constexpr int64_t WIDE_SORT_RAYS = 1000000, WIDE_SORT_TRIS = 100000;
 
 template <bool ANY>
@@ -769,12 +795,17 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
     int *flag = nullptr;
     char *ws = nullptr;
     std::unique_lock<std::mutex> ws_lock;
-    // The wide walk is sorted less: only large incoherent batches gain.
     // (With a negative tmin every ray of it would walk in the reference's
     // order, which the binary walk's kernels do faster.)
     const bool wide = wide_chosen(T) && (s->view.flat || (s->view.wide && tmin >= 0.0f)) && !(T.trace_util && !fixed) &&
                       n < (int64_t)0xf0000000;
-    const int64_t sort_min = !wide ? 4096 : s->view.n_tris < WIDE_SORT_TRIS ? INT64_MAX : ANY ? 2 * WIDE_SORT_RAYS : WIDE_SORT_RAYS;
+    // The wide walk is sorted less: only large batches gain.
+    const bool by_dir = T.ray_sort == 5 && !ANY, cells = s->view.n_tris >= WIDE_SORT_TRIS;
+    const int64_t sort_min = !wide               ? 4096
+                             : s->view.flat      ? INT64_MAX
+                             : cells             ? (ANY ? 2 : 1) * WIDE_SORT_RAYS
+                             : by_dir            ? 4 * WIDE_SORT_RAYS
+                                                 : INT64_MAX;
     if ((T.ray_sort == 4 || T.ray_sort == 5) && n >= sort_min) {
         // the library's radix sort: keys, keys2, values, values2, flag, tile histograms, chunk totals
         const size_t plane = ((size_t)n * 4 + 255) & ~(size_t)255;
@@ -807,8 +838,9 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         const unsigned gn = (unsigned)((n + 255) / 256);
         // mode 5: flag, then the direction range of a coherent batch, in the flag's 256-byte slot;
         // closest-hit calls only (any-hit walks stop at the first hit and do not pay for the sort)
-        float *box = (T.ray_sort == 5 && !ANY && !wide) ? reinterpret_cast<float *>(flag + 1) : nullptr;
-        hipLaunchKernelGGL(k_coherence, dim3(1), dim3(256), 0, st, s->view, rays, n, 0.02f, flag, box);
+        float *box = by_dir ? reinterpret_cast<float *>(flag + 1) : nullptr;
+        hipLaunchKernelGGL(k_coherence, dim3(1), dim3(256), 0, st, s->view, rays, n, 0.02f, flag, box,
+                           !wide ? 0 : cells ? 1 : 2);
         hipLaunchKernelGGL(k_bin_keys, dim3(gn), dim3(256), 0, st, s->view, rays, n, (const int *)flag, keys, vals, 1,
                            (const float *)box);
         for (int pass = 0; pass < 2; ++pass) {
