@@ -923,7 +923,7 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
         int32_t rc = ray_counter(&next);
         if (rc) return rc;
         unsigned pgrid = (unsigned)std::min<int64_t>(grid, (int64_t)device_cu_count() * T.persistent_blocks_per_cu);
-        hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, next);
+        if (!wide) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, next);
         const int nl = std::min(std::max(1, (int)s->view.depth), T.lds_stack_entries);
         const bool util = T.trace_util != 0 && !fixed;
         const int fetch = fetch_lanes(T, wide);
@@ -933,6 +933,10 @@ static int32_t launch_trace(const rm_scene *s, const float *rays, int64_t n, flo
             const uint32_t per = wide_per_wave((uint32_t)n, most, s->view.flat);
             const uint32_t waves = (uint32_t)std::min<int64_t>(most, (n + per - 1) / per);
             pgrid = (waves + TRACE_BLOCK / 64 - 1) / (TRACE_BLOCK / 64);
+            // the waves make no claims when they start with all rays: one
+            // launch less, which a few rays feel (1 ray, 12 triangles: 11.4 -> 8.9 us)
+            if ((int64_t)pgrid * (TRACE_BLOCK / 64) * per < n)
+                hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, st, next);
             hipLaunchKernelGGL(k_trace_wide<ANY>, dim3(pgrid), dim3(TRACE_BLOCK), wide_lds_bytes(s->view.depth), st,
                                s->view, rays, (uint32_t)n, tmin, t0, aim_dev, t_out, id_out, occ, next, per,
                                fetch, (const uint32_t *)order, (const int *)flag, T.walk_phases);

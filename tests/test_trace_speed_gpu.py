@@ -2,6 +2,7 @@
 of the binary tree (trace variant 3, four triangles a step) at the settings
 that suit it, which the default has to come near at least."""
 import contextlib
+import time
 
 import numpy as np
 import pytest
@@ -50,11 +51,15 @@ def both(scene, rays, binary=BINARY, **kw):
         return own, ms(run)
 
 
-def make(v):
+def describe(v):
     v = np.ascontiguousarray(v, np.float32)
     m = rm._lib.RmMaterial(roughness=0.8, opacity=1.0, ior=1.0, albedo_tex=-1, normal_tex=-1, emissive_tex=-1, specular_tex=-1)
     k = len(v)
-    desc, keep = make_desc(v, np.zeros((k, 3, 2)), np.zeros(k), np.zeros(k), [m], [])
+    return make_desc(v, np.zeros((k, 3, 2)), np.zeros(k), np.zeros(k), [m], [])
+
+
+def make(v):
+    desc, keep = describe(v)
     S = rm.Scene(desc)
     S.arrays = keep
     return S
@@ -101,6 +106,23 @@ def test_long_directions(dev, length):
     assert own < 1.3 * binary, (own, binary)
 
 
+@pytest.mark.parametrize("tris", [2, 12, 300])
+def test_one_ray(dev, tris):
+    """The smallest call: its launches are all that it costs."""
+    S = make(soup(tris, 5, 0.3))
+    r = uniform(1, dev)
+    t, i = torch.empty(1, device=dev), torch.empty(1, device=dev, dtype=torch.int32)
+
+    def many():
+        for _ in range(200):
+            S.trace_closest(r, t_out=t, id_out=i)
+
+    own = ms(many)
+    with tuned(BINARY):
+        binary = ms(many)
+    assert own < binary, (own, binary)
+
+
 def camera(side, dev):
     x = (torch.arange(side, device=dev) + 0.5) / side - 0.5
     d = torch.stack([x[None, :].expand(side, side), x[:, None].expand(side, side), torch.full((side, side), 0.8, device=dev)], -1)
@@ -124,5 +146,5 @@ def test_shuffled_camera(dev, tris, side):
     with tuned({rm.TUNE_RAY_SORT: 0}):
         unsorted, rows = ms(lambda: S.trace_closest(q)), ms(lambda: S.trace_closest(r))
     own, image = ms(lambda: S.trace_closest(q)), ms(lambda: S.trace_closest(r))
-    assert own < 0.97 * unsorted, (own, unsorted)
+    assert own < 0.95 * unsorted, (own, unsorted)
     assert image < 1.08 * rows, (image, rows)
