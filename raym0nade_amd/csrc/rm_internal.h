@@ -178,6 +178,13 @@ int32_t launch_mip_build(const rm_scene *s, int t, hipStream_t st);
 // Puts a small scene's rejection records (wide.h) behind its triangles;
 // returns their offset in bytes, 0 for other scenes.
 size_t append_flat(HostScene &h);
+// What the four-wide tree needs to know of a scene as a whole (wide.hip):
+// before the upload, which takes some of it along.  n_big: -1 if unknown.
+struct WideCore {
+    double mid[3], reach, big;
+    int n_big;
+};
+WideCore wide_core(HostScene &h);
 // The four-wide tree of an uploaded scene (wide.h); waits for it.
-int32_t build_wide(rm_scene *s, size_t flat);
+int32_t build_wide(rm_scene *s, size_t flat, const WideCore &core);
 }  // namespace rm

@@ -597,8 +597,9 @@ extern "C" int32_t rm_scene_create(const rm_scene_desc *desc, rm_scene **out) {
     HostScene &h = s->host;
 #define UP(buf, vec) \
     if ((st = s->buf.upload(h.vec.data(), h.vec.size() * sizeof(h.vec[0])))) { delete s; return st; }
-    UP(nodes, pairs);
+    const WideCore core = wide_core(h);
     const size_t flat = append_flat(h);
+    UP(nodes, pairs);
     UP(tris, tris);
     UP(shade, shade);
     UP(mats, mats);
@@ -639,7 +640,7 @@ extern "C" int32_t rm_scene_create(const rm_scene_desc *desc, rm_scene **out) {
     v.sky_w = h.sky_w;
     v.sky_h = h.sky_h;
     v.n_mats = (int32_t)h.mats.size();
-    if ((st = build_wide(s, flat))) { delete s; return st; }
+    if ((st = build_wide(s, flat, core))) { delete s; return st; }
     rm_scene_info &I = s->info;
     I.n_tris = h.n;
     I.n_nodes = h.n_nodes;

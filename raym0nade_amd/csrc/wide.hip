@@ -9,6 +9,7 @@
 // slot of its first would-be descendant.
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 
 #include "rm_internal.h"
 #include "wide.h"
@@ -68,13 +69,45 @@ __device__ __forceinline__ uint32_t flag_children(const double (&v)[4], const bo
     return flags;
 }
 
-__global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__ bin, TriRec *__restrict__ tris,
-                                                    const TriShade *__restrict__ shade, WideNode *__restrict__ out,
-                                                    uint32_t off, int level, int step, uint32_t child_off, float lx,
-                                                    float ly, float lz, double scale, double reach, double big,
-                                                    uint32_t *__restrict__ found) {
-    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= (1u << level)) return;
+// |e2|, infinite where the reference's rejection bounds nothing because the
+// square of |e1| leaves the float range, 0 for a triangle that is never hit.
+__host__ __device__ inline double growth_edge(const TriRec &T) {
+    double l1 = 0.0, l2 = 0.0;
+    for (int a = 0; a < 3; ++a) {
+        l1 += (double)T.e1[a] * T.e1[a];
+        l2 += (double)T.e2[a] * T.e2[a];
+    }
+    if (!(l1 > 0.0 && l2 >= 0.0)) return 0.0;
+    return l1 > 1e-30 ? sqrt(l2) : INFINITY;
+}
+
+// What the records of all levels are made from.
+struct WideBuild {
+    const PairNode *bin;
+    TriRec *tris;
+    const TriShade *shade;
+    WideNode *out;
+    float lo[3];
+    double scale, reach, big;
+    uint32_t *found;    // the large triangles: their number and slots, unless known
+    uint32_t *host;     // where the number found goes in the end
+};
+// A kept level: its nodes are at `off`, the next kept one's at `child`.
+struct WideLevel {
+    int32_t level, step;
+    uint32_t off, child;
+};
+
+// The record of node j of a level.
+__device__ __forceinline__ void wide_node(const WideBuild &A, const WideLevel &L, uint32_t j) {
+    const PairNode *bin = A.bin;
+    TriRec *tris = A.tris;
+    const TriShade *shade = A.shade;
+    WideNode *out = A.out;
+    const float lo[3] = {A.lo[0], A.lo[1], A.lo[2]};
+    const double scale = A.scale, big = A.big;
+    const int level = L.level;
+    if (level == 0 && A.host) *A.host = A.found[0];  // the last level
     // what heap node w = 2^level + j is: follow its bits from the root
     const uint32_t w = (1u << level) + j;
     uint32_t u = 1u, leaf = 0u;
@@ -92,7 +125,6 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
     for (int k = 0; k < 4; ++k) B.used[k] = false;
     double v[4] = {0.0, 0.0, 0.0, 0.0};  // the largest |e2| below each child, scaled
     uint32_t ref;
-    const float lo[3] = {lx, ly, lz};
     if (leaf) {
         const uint32_t first = leaf >> LEAF_SHIFT, c = leaf & LEAF_MASK;
         ref = 0x80000000u | (first << 6) | (c << 2);
@@ -108,17 +140,12 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
                         B.lo[k][a] = fminf(B.lo[k][a], x);  // a NaN is dropped: its triangle is never hit
                         B.hi[k][a] = fmaxf(B.hi[k][a], x);
                     }
-                double l1 = 0.0, l2 = 0.0;
-                for (int a = 0; a < 3; ++a) {
-                    l1 += (double)tris[i].e1[a] * tris[i].e1[a];
-                    l2 += (double)tris[i].e2[a] * tris[i].e2[a];
-                }
-                // (|e1|'s square may leave the float range in the reference's
-                // rejection, which then bounds nothing)
-                const double l = l1 > 1e-30 || l1 == 0.0 ? sqrt(l2) : INFINITY;
-                if (l > big) {  // found[0] of them, the first ones' slots behind
-                    const uint32_t q = atomicAdd(found, 1u);
-                    if (q < MAX_BIG) found[1 + q] = i;
+                const double l = growth_edge(tris[i]);
+                if (l > big) {
+                    if (A.found) {  // found[0] of them, the first ones' slots behind
+                        const uint32_t q = atomicAdd(A.found, 1u);
+                        if (q < MAX_BIG) A.found[1 + q] = i;
+                    }
                 } else {
                     v[k] = fmax(v[k], l * scale);
                 }
@@ -128,8 +155,9 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
             B.used[k] = B.lo[k][0] <= B.hi[k][0] && B.lo[k][1] <= B.hi[k][1] && B.lo[k][2] <= B.hi[k][2];
         }
     } else {
+        const int step = L.step;
         const uint32_t cj = step == 1 ? 2u * j : 4u * j;
-        ref = child_off + cj;
+        ref = L.child + cj;
         const PairNode P = bin[w];
         for (int s = 0; s < 2; ++s) {
             if (step == 1) {
@@ -173,14 +201,36 @@ __global__ __launch_bounds__(256) void k_wide_build(const PairNode *__restrict__
             if (B.used[k]) far[a] = fmax(far[a], ((double)B.hi[k][a] - lo[a]) * scale - org[a]);
     const double d = sqrt(far[0] * far[0] + far[1] * far[1] + far[2] * far[2]) + 1.0;
     double e;
-    const uint32_t flags = flag_children(v, B.used, d, reach, e);
+    const uint32_t flags = flag_children(v, B.used, d, A.reach, e);
     const uint32_t all = (half_up(fmax(fmax(v[0], v[1]), fmax(v[2], v[3]))) + 7u) >> 3;
-    uint4 *o = reinterpret_cast<uint4 *>(out + (off + j));
+    uint4 *o = reinterpret_cast<uint4 *>(out + (L.off + j));
     o[0] = make_uint4(pl[0][0], pl[0][1], pl[0][2], pl[0][3]);
     o[1] = make_uint4(pl[1][0], pl[1][1], pl[1][2], pl[1][3]);
     o[2] = make_uint4(pl[2][0], pl[2][1], pl[2][2], pl[2][3]);
     o[3] = make_uint4((uint32_t)org[0] | ((uint32_t)org[1] << 16),
                       (uint32_t)org[2] | (half_up(e) << 16), half_up(d) | (all << 16) | (flags << 28), ref);
+}
+
+__global__ __launch_bounds__(256) void k_wide_build(WideBuild A, WideLevel L) {
+    const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+    if (j < (1u << L.level)) wide_node(A, L, j);
+}
+
+// All levels of a small tree in one block, children first.  A scene of
+// 1000 triangles is made in 161 us with it, in 214 with a launch a level, and in
+// 113 without the tree.
+constexpr int SMALL_LEVELS = 6;  // levels of at most 2^10 nodes
+struct WideLevels {
+    WideLevel l[SMALL_LEVELS];
+    int32_t n;
+};
+__global__ __launch_bounds__(1024) void k_wide_build_small(WideBuild A, WideLevels W) {
+    for (int i = W.n - 1; i >= 0; --i) {
+        const WideLevel L = W.l[i];
+        if (threadIdx.x < (1u << L.level)) wide_node(A, L, threadIdx.x);
+        __threadfence_block();
+        __syncthreads();
+    }
 }
 
 // The walks' range: coordinates that are finite and whose scaling stays in
@@ -197,31 +247,42 @@ static bool wide_range(const HostScene &h, float &ext, float &mag) {
 
 // Where most triangles lie, whatever a few far ones (a ground) span: the mean
 // of up to 1024 of them and the side of a uniform distribution of their spread.
-// big: BIG_EDGES times their median |e2|.
-constexpr double BIG_EDGES = 16.0;
-static double wide_core(const HostScene &h, double (&mid)[3], double &big) {
+// big: 16 times their median |e2|.  A scene of so few triangles has its larger
+// ones' slots (at most MAX_BIG, else none) in the record of the heap's node 0,
+// which no walk reads; k_wide_build finds those of others.
+WideCore wide_core(HostScene &h) {
     const int64_t n = std::min<int64_t>(h.n, 1024);
-    double reach = 0.0;
+    WideCore c;
+    c.reach = 0.0;
     for (int a = 0; a < 3; ++a) {
         double s = 0.0, q = 0.0, m = 0.0;
-        const double c = h.root_lo[a];
+        const double l = h.root_lo[a];
         for (int64_t i = 0; i < n; ++i) {
-            const double x = (double)h.tris[i * h.n / n].p[a] - c;
+            const double x = (double)h.tris[i * h.n / n].p[a] - l;
             if (!(fabs(x) < 1e30)) continue;
             s += x, q += x * x, m += 1.0;
         }
-        mid[a] = c + (m > 0.0 ? s / m : 0.0);
-        if (m > 0.0) reach = std::max(reach, sqrt(std::max(0.0, 12.0 * (q / m - s / m * (s / m)))));
+        c.mid[a] = l + (m > 0.0 ? s / m : 0.0);
+        if (m > 0.0) c.reach = std::max(c.reach, sqrt(std::max(0.0, 12.0 * (q / m - s / m * (s / m)))));
     }
-    std::vector<float> e((size_t)n);
-    for (int64_t i = 0; i < n; ++i) {
-        const float *v = h.tris[i * h.n / n].e2;
-        const float q = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-        e[(size_t)i] = q == q ? q : 0.0f;
+    std::vector<double> e((size_t)n);
+    for (int64_t i = 0; i < n; ++i) e[(size_t)i] = growth_edge(h.tris[i * h.n / n]);
+    std::vector<double> o(e);
+    std::nth_element(o.begin(), o.begin() + n / 2, o.end());
+    c.big = 16.0 * o[(size_t)(n / 2)];
+    c.n_big = h.n == n ? 0 : -1;
+    if (c.n_big == 0) {
+        uint32_t *slots = reinterpret_cast<uint32_t *>(h.pairs.data()) + 1;
+        for (int64_t i = 0; i < n && c.n_big >= 0; ++i)
+            if (e[(size_t)i] > c.big) {
+                if (c.n_big == (int)MAX_BIG)
+                    c.n_big = -2;
+                else
+                    slots[c.n_big++] = (uint32_t)i;
+            }
+        if (c.n_big < 0) c.n_big = 0, c.big = INFINITY;  // too many: the tree bounds them all
     }
-    std::nth_element(e.begin(), e.begin() + n / 2, e.end());
-    big = BIG_EDGES * sqrt((double)e[(size_t)(n / 2)]);
-    return reach;
+    return c;
 }
 
 // A flat scene's records follow its triangles in their buffer: no kernel and
@@ -264,7 +325,7 @@ size_t append_flat(HostScene &h) {
 // more (a run's reference), coordinates outside wide_range, and sizes that
 // WIDE_SCENE excludes.  flat: where
 // append_flat put the records, or 0.
-int32_t build_wide(rm_scene *s, size_t flat) {
+int32_t build_wide(rm_scene *s, size_t flat, const WideCore &core) {
     SceneView &v = s->view;
     v.wide = nullptr;
     v.flat = 0;
@@ -280,44 +341,60 @@ int32_t build_wide(rm_scene *s, size_t flat) {
         v.flat_tris = reinterpret_cast<const FlatTri *>(s->tris.as<char>() + flat);
         return RM_OK;
     }
-    double mid[3];
-    double big;
-    const double reach = wide_core(h, mid, big);
-    if (!(WIDE_ERR * reach <= WIDE_SCENE)) return RM_OK;
+    if (!(WIDE_ERR * core.reach <= WIDE_SCENE)) return RM_OK;
     const int e = (int)floor(log2(30000.0 / (double)ext));
     const double scale = ldexp(1.0, e);
     for (int a = 0; a < 3; ++a) v.wide_lo[a] = (float)((double)h.root_lo[a] - 1000.0 / scale);
     v.wide_scale = (float)scale;
     v.wide_rscale = (float)(1.0 / scale);
-    for (int a = 0; a < 3; ++a) v.wide_mid[a] = (float)((mid[a] - v.wide_lo[a]) * scale);
-    v.wide_reach = (float)(reach * scale);
+    for (int a = 0; a < 3; ++a) v.wide_mid[a] = (float)((core.mid[a] - v.wide_lo[a]) * scale);
+    v.wide_reach = (float)(core.reach * scale);
     const int leaf_level = h.depth - 1;  // the deepest leaves' level
-    struct Level { int level, step; uint32_t off; };
-    std::vector<Level> levels;
+    std::vector<WideLevel> levels;
     uint32_t total = 0;
     for (int l = 0; l <= leaf_level;) {
         const int step = l == 0 && (leaf_level & 1) ? 1 : 2;
-        levels.push_back(Level{l, step, total});
-        total += std::max(4u, 1u << l);
+        levels.push_back(WideLevel{l, step, total, total + std::max(4u, 1u << l)});
+        total = levels.back().child;
         l += step;
     }
-    const int32_t rc = s->wide.alloc((size_t)(total + 1) * sizeof(WideNode));
+    const int32_t rc = s->wide.alloc((size_t)total * sizeof(WideNode));
     if (rc) return rc;
-    uint32_t *found = reinterpret_cast<uint32_t *>(s->wide.as<WideNode>() + total), got = 0;
+    static_assert((1 + MAX_BIG) * sizeof(uint32_t) <= sizeof(PairNode), "room for the slots in node 0's record");
+    uint32_t *found = s->nodes.as<uint32_t>();
+    double big = core.big;
+    uint32_t got = 0, *pin = nullptr;
+    std::unique_lock<std::mutex> lock;
+    if (core.n_big < 0) {
+        // the number found comes back in pinned memory, kept until the process
+        // ends (a copy's wait takes 40 us more); one scene at a time
+        static std::mutex mu;
+        static uint32_t *kept = nullptr;
+        lock = std::unique_lock<std::mutex>(mu);
+        if (!kept) RM_HIP(hipHostMalloc((void **)&kept, sizeof(uint32_t), hipHostMallocPortable));
+        pin = kept;
+    }
     while (true) {
-        RM_HIP(hipMemset(found, 0, sizeof(WideNode)));
-        for (size_t i = levels.size(); i-- > 0;) {  // children first: their E
-            const Level &L = levels[i];
-            const uint32_t child = i + 1 < levels.size() ? levels[i + 1].off : 0u;
-            hipLaunchKernelGGL(k_wide_build, dim3(((1u << L.level) + 255) / 256), dim3(256), 0, nullptr, v.nodes,
-                               s->tris.as<TriRec>(), v.shade, s->wide.as<WideNode>(), L.off, L.level, L.step, child,
-                               v.wide_lo[0], v.wide_lo[1], v.wide_lo[2], scale, reach, big, found);
+        const WideBuild A{v.nodes, s->tris.as<TriRec>(), v.shade, s->wide.as<WideNode>(),
+                          {v.wide_lo[0], v.wide_lo[1], v.wide_lo[2]}, scale, core.reach, big,
+                          core.n_big < 0 ? found : nullptr, pin};
+        if (leaf_level <= 10) {
+            WideLevels W{};
+            W.n = (int32_t)levels.size();
+            std::copy(levels.begin(), levels.end(), W.l);
+            hipLaunchKernelGGL(k_wide_build_small, dim3(1), dim3(1024), 0, nullptr, A, W);
+        } else {
+            for (size_t i = levels.size(); i-- > 0;)  // children first: their E
+                hipLaunchKernelGGL(k_wide_build, dim3(((1u << levels[i].level) + 255) / 256), dim3(256), 0, nullptr, A,
+                                   levels[i]);
         }
         RM_HIP(hipGetLastError());
-        // waits: the caller may use the scene on any stream next
-        RM_HIP(hipMemcpy(&got, found, sizeof(got), hipMemcpyDeviceToHost));
+        // the caller may use the scene on any stream next
+        RM_HIP(hipStreamSynchronize(nullptr));
+        got = core.n_big < 0 ? *pin : (uint32_t)core.n_big;
         if (got <= MAX_BIG) break;
-        big = INFINITY;  // too many: the tree bounds them all
+        big = INFINITY;  // as in wide_core
+        RM_HIP(hipMemset(found, 0, sizeof(PairNode)));
     }
     v.n_big = (int32_t)got;
     v.big = found + 1;

@@ -123,6 +123,25 @@ def test_one_ray(dev, tris):
     assert own < binary, (own, binary)
 
 
+def test_scene_creation(dev):
+    """A small scene with its four-wide tree, against one whose place excludes that."""
+    near = soup(1000, 6, 0.1)
+    far = (near + np.float32(2e4)).astype(np.float32)
+
+    def seconds(v):
+        desc, keep = describe(v)
+        best = float("inf")
+        for _ in range(50):
+            t0 = time.perf_counter()
+            rm.Scene(desc)
+            best = min(best, time.perf_counter() - t0)
+        return best
+
+    seconds(near)
+    own, bare = seconds(near), seconds(far)
+    assert own < 1.6 * bare, (own, bare)
+
+
 def camera(side, dev):
     x = (torch.arange(side, device=dev) + 0.5) / side - 0.5
     d = torch.stack([x[None, :].expand(side, side), x[:, None].expand(side, side), torch.full((side, side), 0.8, device=dev)], -1)
