@@ -71,7 +71,7 @@ __device__ __forceinline__ void tile_box(int x, int y, int r, int w, int h, int 
 // tile (a global atomic per pixel and tile, as before, cost more than the
 // rest: 716 -> 80 us at 1080p, CoC 8, with the table of roots).
 __global__ __launch_bounds__(DB) void k_dof_src(const float *__restrict__ pos, int w, int h, float focus, float coc,
-                                               V3 cam, int ntx, int nty, DofSrc *__restrict__ src,
+                                               V3 cam, int ntx, DofSrc *__restrict__ src,
                                                uint64_t *__restrict__ key, uint32_t *__restrict__ tile_count) {
     __shared__ float root[ROOTS];
     __shared__ uint32_t cnt[NEAR_W * NEAR_W];
@@ -283,7 +283,7 @@ int32_t rm::dof_launch(rm_frame *f, const float *in, float *out, hipStream_t st)
     hipLaunchKernelGGL(k_dof_zero, dim3((nt + DB - 1) / DB), dim3(DB), 0, st, count, nt);
     V3 cam{f->dof_cam[0], f->dof_cam[1], f->dof_cam[2]};
     hipLaunchKernelGGL(k_dof_src, dim3(nt), dim3(DB), 0, st, f->buf[RM_BUF_POSITION].as<float>(), w, h, f->dof_focus,
-                       f->dof_coc, cam, ntx, nty, src, key, count);
+                       f->dof_coc, cam, ntx, src, key, count);
     hipLaunchKernelGGL(k_dof_scan, dim3(1), dim3(1024), 0, st, (const uint32_t *)count, nt, off, cursor);
     RM_HIP(hipGetLastError());
     uint32_t total = 0;

@@ -141,7 +141,7 @@ struct Tuning {
     int render_blocks_per_cu = 4; // resident blocks per CU of the persistent bounce kernel
     int adjoint_split = 4;        // lanes per pixel of the adjoint kernel
     int kernel_timing = 0;        // record HIP events around the trace kernels (rm_last_trace_ms)
-    int render_min_waves = 1;     // 1 or 4: register cap of the shading and NEE kernels
+    int render_min_waves = 1;     // 1, 3 or 4: register cap of the shading and NEE kernels
     int lds_stack_entries = 10;   // trace variant 3: walk-stack entries per lane kept in LDS (160 KiB at 8 blocks/CU)
     int tris_per_step = 0;        // trace variant 3: triangles tested per step (0: the four-wide walk)
     int nee_split = 2;            // render: shadow rays of light samples in their own passes (2: deep trees)

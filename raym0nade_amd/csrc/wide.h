@@ -56,14 +56,12 @@
 // 10% of scenes of small spheres on a ground.)  What bounds it now: the same data path
 // (94% busy), then the vector ALUs.
 #pragma once
-#include <type_traits>
 #include "traverse.h"
 
 namespace rm {
 
 constexpr int WALK_WIDE = 6;     // walk kind of the render's inlined walks (beside 0, 1, 2, 4 triangles per step)
 constexpr int WALK_FLAT = 7;     // walk kind: every triangle of a flat scene, else the reference-order walk
-constexpr int WIDE_LEVELS = 14;  // nodes on a path of a four-wide tree over fewer than 2^25 triangles, at most
 constexpr uint32_t WIDE_NONE = 0xffffffffu;
 
 // A group of up to four sibling children still to visit, two words: x = the
@@ -73,9 +71,9 @@ constexpr uint32_t WIDE_NONE = 0xffffffffu;
 // at most one group per level of the tree, and keeps its newest in registers.
 constexpr uint32_t GROUP_T = 0xfffff800u;
 
-// The walk's older groups.  WideLds: in the block's dynamic LDS (blocks of
-// WALK_BLOCK lanes; the launch provides wide_lds_bytes), so that a wave's
-// accesses to one entry are contiguous.  WidePrivate: in per-lane scratch.
+// The walk's older groups, in the block's dynamic LDS (blocks of WALK_BLOCK
+// lanes; the launch provides wide_lds_bytes), so that a wave's accesses to one
+// entry are contiguous.
 struct WideLds {
     uint2 *col;
     __device__ __forceinline__ void bind() {
@@ -84,12 +82,6 @@ struct WideLds {
     }
     __device__ __forceinline__ void put(int i, uint32_t x, uint32_t y) { col[i * WALK_BLOCK] = make_uint2(x, y); }
     __device__ __forceinline__ uint2 get(int i) const { return col[i * WALK_BLOCK]; }
-};
-struct WidePrivate {
-    uint2 e[WIDE_LEVELS];
-    __device__ __forceinline__ void bind() {}
-    __device__ __forceinline__ void put(int i, uint32_t x, uint32_t y) { e[i] = make_uint2(x, y); }
-    __device__ __forceinline__ uint2 get(int i) const { return e[i]; }
 };
 // Entries and bytes of dynamic LDS per block for the walk of a tree of
 // `depth` binary levels (leaves included).
@@ -229,9 +221,8 @@ __device__ __forceinline__ uint32_t bit_select(uint32_t mask, uint32_t a, uint32
 // runs wait in l while the lane goes on to its next nodes, until a second
 // leaf's runs come up.  So a wave can take steps of one kind with most of its
 // lanes, whichever kind its lanes came to first.
-template <class Stack>
 struct WideWalker {
-    Stack stk;
+    WideLds stk;
     int sp;             // groups in stk
     uint32_t cur;       // the node to visit next, or WIDE_NONE
     uint32_t gx, gy;    // newest group
@@ -519,10 +510,15 @@ struct RefWalker {
 // reference's own order.
 //
 // The rejection works on the unscaled values a, u a and v a from the line's
-// moment (25 instructions a triangle, the exact test takes 66).  Its own
-// roundings and those of the exact test, whose accepted u and v may lie
-// outside [0, 1] by theirs, stay below 16 eps |d| (|e1| + |e2|) (|o| + |v0| +
-// |e1|) each; twice their sum is allowed (FLAT_ERR, eps = 2^-24).
+// moment (25 instructions a triangle, the exact test takes 66).  With eps =
+// 2^-24: u a and v a are off here by at most 8 eps |d| |e| |o| + 7 eps |d| |e|
+// |v0|, e being e2 or e1, and in the exact test, whose accepted u and v may lie
+// outside [0, 1] by that, by 5.2 eps |d| |e| (|o| + |v0|); a by 4 and 5.2 eps |d|
+// |e1| |e2|, and rounding u, v and their sum by 5 more.  Together at most 13.2 eps
+// |d| (|e1| + |e2|) (|o| + |v0|) + 14.2 eps |d| |e1| |e2|.  With coordinates of at
+// most m, |v0| is at most 1.74 m and |e1| |e2| at most 1.74 m (|e1| + |e2|), so this
+// is below eps |d| (|e1| + |e2|) (13.2 |o| + 48 m); 64 |o| + 192 m are allowed
+// (FLAT_ERR, flat_b = 3 m).
 //
 // FLAT_MAX is the masks' width.  Closest hits of 2M rays among 12 / 36 / 64
 // triangles take 41 / 80 / 125 us, in the binary walk 616 / 645 / 681, of 20k
@@ -611,10 +607,10 @@ __device__ __forceinline__ bool hit_sure(const SceneView &S, V3 o, V3 d, float t
 }
 
 // The whole wide walk of one ray, for kernels that do more than traversal.
-// Same contract as trace_walk.  LDSW: the kernel provides wide_lds_bytes.
-template <bool ANY, bool LDSW>
+// Same contract as trace_walk; the kernel provides wide_lds_bytes.
+template <bool ANY>
 __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, float tmin, float &tmax, float aim) {
-    WideWalker<typename std::conditional<LDSW, WideLds, WidePrivate>::type> w;
+    WideWalker w;
     WideRay r;
     RefWalker ref;
     w.stk.bind();
@@ -657,7 +653,7 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
 // wave: 10k rays 223 / 241 / 258 / 278 us, 100k rays 571 / 377 / 344 / 339 us).
 // The rays of a flat scene cost the same, so a wave takes whole batches, its
 // whole share at the start where that is at most 512: claims are atomic adds
-// to one address, 12 ns each, and 64 rays a claim held 2M closest hits among
+// to one address, 12 ns each on the traces' 64-bit counter, and 64 rays a claim held 2M closest hits among
 // 36 triangles to 392 us (80 so, and 302 for 8M).
 __host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bool flat) {
     if (flat) {
@@ -684,8 +680,8 @@ __host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bo
 // lanes then check and store their results together.  Each iteration takes
 // one kind of step: runs when at least phases / 64 of the walking lanes have
 // one, else nodes.  Every wave leaves when its rays are used up and its lanes
-// are done.  (Waves that all begin with an atomic on one address wait 6 ns for
-// each other: 50 us for a launch of 8192 with little or nothing to do.)
+// are done.  (Waves that all begin with an atomic on one address wait 6 ns
+// for each other on the renders' 32-bit counters: 50 us for a launch of 8192 with little or nothing to do.)
 template <bool ANY, class Src, class Count>
 __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, float tmin, int fetch_min, int phases) {
     const uint32_t lane = threadIdx.x & 63u;
@@ -696,7 +692,7 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
     if (at >= n) return;
     uint32_t end = at + per < n ? at + per : n;
     bool more = begun < n;
-    WideWalker<WideLds> w;
+    WideWalker w;
     RefWalker ref;
     WideRay r;
     w.stk.bind();
@@ -788,8 +784,9 @@ __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, f
 // with TPS triangles per step.
 template <bool ANY, bool LDSW = true, int TPS = 0>
 __device__ __forceinline__ int32_t scene_walk(const SceneView &S, const RayPre &r, float tmin, float &tmax, float aim) {
+    static_assert(TPS != WALK_WIDE || LDSW, "the wide walk's groups are in LDS");
     if constexpr (TPS == WALK_WIDE)
-        return wide_walk<ANY, LDSW>(S, r.o, r.d, tmin, tmax, aim);
+        return wide_walk<ANY>(S, r.o, r.d, tmin, tmax, aim);
     else if constexpr (TPS == WALK_FLAT) {
         if (S.flat) {
             float tm = tmax, t2 = tmax;

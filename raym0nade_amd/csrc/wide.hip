@@ -358,8 +358,9 @@ int32_t build_wide(rm_scene *s, size_t flat, const WideCore &core) {
         total = levels.back().child;
         l += step;
     }
+    // a scene that fits without the tree walks the binary one
     const int32_t rc = s->wide.alloc((size_t)total * sizeof(WideNode));
-    if (rc) return rc;
+    if (rc) return rc == RM_ERR_OOM ? RM_OK : rc;
     static_assert((1 + MAX_BIG) * sizeof(uint32_t) <= sizeof(PairNode), "room for the slots in node 0's record");
     uint32_t *found = s->nodes.as<uint32_t>();
     double big = core.big;

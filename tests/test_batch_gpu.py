@@ -50,6 +50,30 @@ def test_batch_equals_single_renders(dev, use_graph):
         assert np.isclose(px, px1, rtol=1e-4, atol=1e-5).all(axis=-1).mean() >= 0.999
 
 
+def moved(g, off):
+    """The generated scene and its camera, shifted."""
+    g.verts[:] = g.verts + np.float32(off)
+    for k in range(3):
+        g.args.position[k] += off
+    return g
+
+
+@pytest.mark.parametrize("last", ["near", "far"])
+def test_batch_of_all_kinds_of_scenes(dev, last):
+    """Scenes tested without a tree, on the four-wide tree, and (far from the
+    origin) on the binary tree only, which then takes the whole batch."""
+    gens = [rm.generate(0, 1), rm.generate(2, 5, grid=1, freq=6, sky_width=64, sky_height=32),
+            rm.generate(2, 6, grid=2, freq=12, sky_width=64, sky_height=32), moved(rm.generate(0, 3), 3e4 if last == "far" else 0.0)]
+    jobs = [(rm.Scene(g), job_args(g, 60 + 8 * i, 52, 8, 8, 7 + i), rm.Frame(60 + 8 * i, 52), 63) for i, g in enumerate(gens)]
+    rm.render_batch(jobs)
+    torch.cuda.synchronize()
+    for S, a, fr, _ in jobs:
+        gb, rad = RC.download_all(fr)
+        gb1, rad1 = RC.gpu_render(S, a)
+        RC.assert_gbuffer_equal(gb, gb1)
+        assert np.isclose(rad, rad1, rtol=1e-4, atol=1e-6).all(axis=-1).mean() >= 0.999
+
+
 def test_serving_batch_with_autotune_equals_single_renders(dev):
     from raym0nade_amd import autotune, workloads
     specs = workloads.batch_specs(6, seed=3, min_log2=5.0, max_log2=6.5)

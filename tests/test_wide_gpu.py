@@ -55,6 +55,8 @@ SCENES = {
     "soup7001": lambda: soup(7001, 10, 0.05), "walls": lambda: walls(9),
     "needles3": lambda: np.concatenate([soup(900, 16, 0.2), needles(3)]),
     "needles12": lambda: np.concatenate([soup(900, 17, 0.2), needles(12)]),
+    # outside the tree's range: far from the origin, and too large
+    "far_off": lambda: (soup(700, 19, 0.2) + np.float32(2e4)).astype(np.float32), "large": lambda: soup(900, 20, 0.2) * np.float32(500),
     "doubled": lambda: np.repeat(soup(700, 11, 0.2), 2, axis=0),
     "twice": lambda: np.concatenate([soup(701, 11, 0.2)] * 2), "thrice": lambda: np.concatenate([soup(501, 11, 0.2)] * 3),
     "twice_flat": lambda: np.concatenate([soup(31, 11, 0.4)] * 2), "thrice_flat": lambda: np.concatenate([soup(21, 11, 0.4)] * 3),
@@ -108,7 +110,7 @@ def test_bit_exact(dev, scene):
     for kind in ("box", "vertices", "edges", "surface", "axis", "far", "length", "odd"):
         r = rays_for(v, kind, n, 17)
         rd = torch.from_numpy(r).to(dev)
-        for tmin, tmax in ((1e-4, np.inf), (0.05, 0.7)) if kind != "odd" else ((1e-4, np.inf),):
+        for tmin, tmax in ((1e-4, np.inf), (0.05, 0.7), (-0.5, np.inf)) if kind != "odd" else ((1e-4, np.inf),):
             t, ids = S.trace_closest(rd, tmin=tmin, tmax=tmax)
             to, io = OS.closest(r, tmin=tmin, tmax=tmax)
             assert np.array_equal(ids.cpu().numpy(), io), (scene, kind, tmin)
@@ -184,6 +186,35 @@ def test_grazing(dev, n, n_big, ext, small, big):
             to, io = OS.closest(few)
             assert np.array_equal(i0[:2000].cpu().numpy(), io)
             assert np.array_equal(t0[:2000].cpu().numpy().view(np.uint32), to.view(np.uint32))
+
+
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_reciprocal(dev, sign):
+    """The corrected reciprocal of the triangle test against the division, for
+    every significand: a = m for a ray (0.25, 0.25, 1) + t (0, 0, -m) and the
+    triangle (0, 0, 0), (1, 0, 0), (0, 1, 0), t = 1 / m."""
+    v = np.float32([[[0, 0, 0], [1, 0, 0], [0, 1, 0]]])
+    if sign < 0:
+        v = v[:, [0, 2, 1]]
+    v = np.ascontiguousarray(v)
+    m = rm._lib.RmMaterial(roughness=0.8, opacity=1.0, ior=1.0, albedo_tex=-1, normal_tex=-1, emissive_tex=-1, specular_tex=-1)
+    desc, keep = make_desc(v, np.zeros((1, 3, 2)), np.zeros(1), np.zeros(1), [m], [])
+    S = rm.Scene(desc)
+    bits = torch.arange(1 << 23, device=dev, dtype=torch.int32) + 0x3f800000
+    x = bits.view(torch.float32)
+    r = torch.zeros(1 << 23, 6, device=dev)
+    r[:, 0] = r[:, 1] = 0.25
+    r[:, 2] = 1.0
+    r[:, 5] = -x
+    t, ids = S.trace_closest(r)
+    want = (1.0 / x.double()).float()  # (of 24 bits, so rounding twice does no harm)
+    assert bool((ids == 0).all())
+    assert torch.equal(t.view(torch.int32), want.view(torch.int32))
+    for scale in (2.0 ** -12, 2.0 ** 20, 2.0 ** 25):
+        r[:, 5] = -x * scale
+        t, ids = S.trace_closest(r, tmin=1e-9)
+        assert bool((ids == 0).all())
+        assert torch.equal((t * scale).view(torch.int32), want.view(torch.int32)), scale
 
 
 @pytest.mark.parametrize("tris", [36, 3001])
