@@ -8,8 +8,9 @@ uniform on the sphere); tmin 1e-4, tmax inf.  One step = one closest-hit
 traversal of both batches, rays resident in HBM.
 
 Also reported: any-hit Mrays/s of the same batches, the traversal kernel's
-roofline (algorithmic bytes per ray priced in the reference traversal order:
-24 + 8 + 24*box_tests + 8*node_visits + 36*triangle_tests), and the oracle's
+roofline (its own bytes beyond L2, from the committed counter passes; beside
+it what the reference's order would read without a cache, 24 + 8 +
+24*box_tests + 8*node_visits + 36*triangle_tests per ray), and the oracle's
 CPU restatement of BVH::rayHit timed on this host on a bounded sample.
 """
 from __future__ import annotations
@@ -202,7 +203,7 @@ def main():
     rm.set_tuning(rm.TUNE_KERNEL_TIMING, 0)
     bytes_per_launch = (algo[("coh", False)] + algo[("inc", False)]) / 2
     dur_per_launch = (np.mean(kt["coh"]) + np.mean(kt["inc"])) / 2 * 1e-3
-    achieved = bytes_per_launch / dur_per_launch / 1e9
+    reference_gbs = bytes_per_launch / dur_per_launch / 1e9
     kernel_name = {0: "k_trace_closest", 2: "k_trace_persistent",
                    3: "k_trace_persistent_lds"}[rm.get_tuning(rm.TUNE_TRACE_VARIANT)]
     if kernel_name == "k_trace_persistent_lds" and rm.get_tuning(rm.TUNE_TRIS_PER_STEP) == 0:
@@ -217,16 +218,20 @@ def main():
             traffic, traffic_launch = tj.get("hbm_bytes_per_launch"), tj.get("launch")
         except (OSError, ValueError):
             traffic = None
-    roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                "traffic_launch": traffic_launch,
-                "kernel": kernel_name, "algorithmic_bytes_per_launch": round(bytes_per_launch),
+    # achieved: the kernel's own bytes beyond L2.  The reference order's reads
+    # are what its walk would need without any cache; the kernel makes others.
+    achieved = traffic / dur_per_launch / 1e9 if traffic else None
+    roofline = {"bound": "hbm", "achieved": round(achieved, 1) if achieved else None, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": round(achieved / HBM_PEAK_GBS, 4) if achieved else None, "traffic": traffic,
+                "traffic_launch": traffic_launch, "kernel": kernel_name,
+                "reference_order_bytes_per_launch": round(bytes_per_launch), "reference_order_gbs": round(reference_gbs, 1),
                 "avg_launch_ms": round(dur_per_launch * 1e3, 4),
                 "launch_ms": {k: round(float(np.mean(v)), 4) for k, v in kt.items()},
                 "reorder_ms": {k: round(float(np.mean(v)), 4) for k, v in rt.items()}}
 
-    # lane utilisation of the persistent LDS walk (untimed calls with the
-    # instrumented kernel; the results are unchanged)
+    # lane utilisation of the binary tree's persistent walk (untimed calls with
+    # its instrumented kernel; the results are unchanged): not of the four-wide
+    # walk, which has no such counts
     if rm.get_tuning(rm.TUNE_TRACE_VARIANT) == 3:
         util = {}
         for name, r in (("coh", r_coh), ("inc", r_inc)):
@@ -235,8 +240,8 @@ def main():
             S.trace_closest(r, t_out=t_out, id_out=id_out)
             util[name] = {k: (round(v, 4) if isinstance(v, float) else v) for k, v in rm.last_trace_util().items()}
             rm.set_tuning(rm.TUNE_TRACE_UTIL, 0)
-        roofline["lane_utilisation"] = util
-        log("[bench] lane utilisation:", {k: (v["interior_util"], v["leaf_util"], v["util"]) for k, v in util.items()})
+        roofline["binary_walk_lane_utilisation"] = util
+        log("[bench] lane utilisation of the binary walk:", {k: (v["interior_util"], v["leaf_util"], v["util"]) for k, v in util.items()})
 
     # measured streaming bandwidth: a plain 1 GiB device copy (1 GiB read + 1 GiB
     # written per launch); also the known-size kernel that scales the
@@ -254,7 +259,8 @@ def main():
     copy_gbs = 2 * (1 << 30) * 5 / (e0.elapsed_time(e1) * 1e-3) / 1e9
     del x, y
     roofline["measured_copy_gbs"] = round(copy_gbs, 1)
-    roofline["frac_of_measured"] = round(achieved / copy_gbs, 4)
+    roofline["frac_of_measured"] = round(achieved / copy_gbs, 4) if achieved else None
+    roofline["reference_order_frac_of_measured"] = round(reference_gbs / copy_gbs, 4)
 
     cpu = None
     if not args.no_cpu:
@@ -647,16 +653,15 @@ def render_roofline(rm, torch, dev, S, a, st, counted, wall):
     ray_bytes = 32 * (n_pri + n_ext) + 25 * n_sh
     other = 60 * st["hits"] + 152 * a.width * a.height
     total = walk_bytes + ray_bytes + other
-    achieved = total / wall / 1e9
+    reference_gbs = total / wall / 1e9  # what the reference's order would read, not what the kernels do
     rays_total = n_pri + n_ext + n_sh
     log(f"[bench] 1080p rays: {rays_total / 1e9:.2f} G ({n_pri} primary, {n_ext} extension, {n_sh} shadow), "
-        f"{rays_total / wall / 1e6:.0f} Mrays/s; algorithmic {total / 1e9:.1f} GB, {achieved:.0f} GB/s")
+        f"{rays_total / wall / 1e6:.0f} Mrays/s; reference order {total / 1e9:.1f} GB, {reference_gbs:.0f} GB/s")
     return {"rays_per_s": round(rays_total / wall, 1), "rays": {"primary": n_pri, "extension": n_ext, "shadow": n_sh},
             "stats": st, "counting_render_matches": same,
-            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
+            "roofline": {"bound": "hbm", "achieved": None, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": None, "traffic": None,
                          "kernel": "whole render (k_primary ... k_finish, FXAA post)",
-                         "algorithmic_bytes_per_frame": round(total),
+                         "reference_order_bytes_per_frame": round(total), "reference_order_gbs": round(reference_gbs, 1),
                          "bytes": {"walks": round(walk_bytes), "rays": round(ray_bytes), "vertices_pixels": round(other)},
                          "walk_counts": {"primary": [pi, pl, pb, pt],
                                          "extension_shadow": [counted["walk_interior"], counted["walk_leaves"],
