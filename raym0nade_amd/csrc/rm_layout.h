@@ -49,10 +49,10 @@ static_assert(sizeof(TriRec) == 48, "TriRec is 48 B");
 // node's origin in scaled coordinates; an empty child has an infinite lower
 // and a zero upper plane.  m[0] = origin x | y << 16, m[1] = origin z | E << 16,
 // m[2] = D | all << 16 | flags << 28, m[3] = reference of child 0 (child k: + k).
-// E: the largest |e2| of the triangles below the children without a flag,
-// scaled; D: the distance from the origin to the farthest corner of the
-// children; both fp16 rounded up.  Flag k: child k holds larger triangles.
-// all: the largest |e2| of all triangles below, an fp16 number's upper 12 bits.
+// E: the largest |e2| of the triangles below the children without a flag, and
+// D: how far from the origin they reach, without those tested before the walk
+// (SceneView::big), scaled, fp16 rounded up.  Flag k: child k holds larger ones.
+// all: as E, of all children, an fp16 number's upper 12 bits.
 struct alignas(64) WideNode {
     uint32_t x[4], y[4], z[4], m[4];
 };

@@ -276,20 +276,18 @@ struct WideWalker {
         y = (y & 0x600u) ? rest : 0u;
     }
 
-    // pad for a ray with parallel axes.  Along such an axis the reference
-    // visits a leaf only when the origin lies within its box, so the distance
-    // there is at most the leaf's size (D once more); and over the runs, which
-    // are smaller than the leaf, the ray drifts by its small component.
+    // pad for a ray with parallel axes, whose planes lie at 2^60 times their
+    // distance.  Over a leaf's runs, which are smaller than the leaf, the ray
+    // also drifts by its small component.
     static __device__ __forceinline__ float par_pad(const WideRay &r, float scale, const float (&cn)[3], uint4 M) {
         const float d[3] = {fabsf(r.d.x), fabsf(r.d.y), fabsf(r.d.z)};
-        float sum = 0.0f, drift = 0.0f;
+        float dist = half_lo(M.z), drift = 0.0f;
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             const bool par = d[a] < T_EPS;
-            sum += par ? 0.0f : fabsf(cn[a]) * d[a];
+            dist = __builtin_fmaf(fabsf(cn[a]), par ? 0x1p-60f : d[a] * scale, dist);
             drift = par ? fmaxf(drift, d[a]) : drift;
         }
-        const float dist = __builtin_fmaf(sum, scale, 2.0f * half_lo(M.z));
         const float pad = -r.err * half_hi(M.y) * dist;
         return M.w & 0x80000000u ? __builtin_fmaf(drift / fmaxf(fmaxf(d[0], d[1]), d[2]), dist, pad) : pad;
     }
@@ -384,11 +382,8 @@ struct WideWalker {
     // first triangle stands, as in the reference; an equal t of another leaf
     // is kept in tie, or -1 there for two such leaves.  tie is memory, touched
     // only then: another register would cost every walk 4%.
-    __device__ __forceinline__ void test(const TriRec *tris, uint32_t i, V3 o, V3 d, float tmin, volatile int32_t &tie) {
-        TriRec T = load_tri(tris, i);
-        // the whole record at once: v0 loaded past the first rejection
-        // would cost a second memory latency
-        asm volatile("" : "+v"(T.p[0]), "+v"(T.p[1]), "+v"(T.p[2]));
+    __device__ __forceinline__ void test(const TriRec *tris, uint32_t i, const TriRec &T, V3 o, V3 d, float tmin,
+                                         volatile int32_t &tie) {
         const float t = tri_test_flat(o, d, V3{T.p[0], T.p[1], T.p[2]}, T.p[3], V3{T.e1[0], T.e1[1], T.e1[2]},
                                       V3{T.e2[0], T.e2[1], T.e2[2]});
         if (tmin < t && t <= t2) {
@@ -423,9 +418,18 @@ struct WideWalker {
             t2 = __uint_as_float(__float_as_uint(tmax) + 1u);
         }
     }
-    // Those that the boxes' growth leaves out.
+    // Those that the boxes' growth leaves out, by scalar loads where a wave's
+    // lanes share the scene.
     __device__ __forceinline__ void test_big(const SceneView &S, V3 o, V3 d, float tmin, volatile int32_t &tie) {
-        for (int k = 0; k < S.n_big; ++k) test(S.tris, S.big[k], o, d, tmin, tie);
+        typedef const __attribute__((address_space(4))) uint32_t scalar_uint;
+        typedef const __attribute__((address_space(4))) float scalar_float;
+        scalar_uint *slots = (scalar_uint *)(uint64_t)S.big;
+        for (int k = 0; k < S.n_big; ++k) {
+            const uint32_t i = slots[k];
+            scalar_float *p = (scalar_float *)(uint64_t)(S.tris + i);
+            const TriRec T{{p[0], p[1], p[2], p[3]}, {p[4], p[5], p[6], p[7]}, {p[8], p[9], p[10], p[11]}};
+            test(S.tris, i, T, o, d, tmin, tie);
+        }
     }
 
     // Tests the first run of l.
@@ -433,7 +437,11 @@ struct WideWalker {
         const uint32_t first = (lx >> 6) & 0x1ffffffu, c = (lx >> 2) & 15u, k = ly & 3u;
         const uint32_t end = first + (c * (k + 1u) >> 2);
         for (uint32_t i = first + (c * k >> 2); i < end; ++i) {
-            test(tris, i, r.o, r.d, tmin, tie);
+            TriRec T = load_tri(tris, i);
+            // the whole record at once: v0 loaded past the first rejection
+            // would cost a second memory latency
+            asm volatile("" : "+v"(T.p[0]), "+v"(T.p[1]), "+v"(T.p[2]));
+            test(tris, i, T, r.o, r.d, tmin, tie);
         }
         drop_first(ly);
         const float lim = wide_limit(tmax);

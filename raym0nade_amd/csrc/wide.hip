@@ -193,16 +193,49 @@ __device__ __forceinline__ void wide_node(const WideBuild &A, const WideLevel &L
         pl[a][2] = h[0] | (h[1] << 16);
         pl[a][3] = h[2] | (h[3] << 16);
     }
-    // D: from the node's origin to the farthest corner of its children, and
-    // one unit more for the roundings of a walk's distance to that origin
-    double far[3] = {0.0, 0.0, 0.0};
-    for (int a = 0; a < 3; ++a)
-        for (int k = 0; k < 4; ++k)
-            if (B.used[k]) far[a] = fmax(far[a], ((double)B.hi[k][a] - lo[a]) * scale - org[a]);
-    const double d = sqrt(far[0] * far[0] + far[1] * far[1] + far[2] * far[2]) + 1.0;
+    // how far from the node's origin each child's triangles reach, the large
+    // ones before the walk left out: over them, and not over the boxes, which
+    // one ground triangle can stretch to the scene's size
+    double far[4] = {0.0, 0.0, 0.0, 0.0}, size = 0.0;
+    for (int k = 0; k < 4; ++k) {
+        if (!B.used[k]) continue;
+        double q = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            const double x = ((double)B.hi[k][a] - lo[a]) * scale - org[a];
+            q += x > 0.0 ? x * x : 0.0;
+        }
+        far[k] = sqrt(q);
+        size = fmax(size, far[k]);
+        if (!leaf) {
+            const WideNode &C = out[ref + k];
+            const double x = (double)(C.m[0] & 0xffffu) - org[0], y = (double)(C.m[0] >> 16) - org[1],
+                         z = (double)(C.m[1] & 0xffffu) - org[2];
+            far[k] = fmin(far[k], sqrt(x * x + y * y + z * z) + (double)__builtin_bit_cast(_Float16, (unsigned short)(C.m[2] & 0xffffu)));
+        } else {
+            const uint32_t first = leaf >> LEAF_SHIFT, c = leaf & LEAF_MASK;
+            double reach = 0.0;
+            for (uint32_t i = first + (c * k >> 2); i < first + (c * (k + 1) >> 2); ++i) {
+                if (growth_edge(tris[i]) > big) continue;
+                for (int p = 0; p < 3; ++p) {
+                    q = 0.0;
+                    for (int a = 0; a < 3; ++a) {
+                        const double x = ((double)shade[i].v[p][a] - lo[a]) * scale - org[a];
+                        q += x * x;
+                    }
+                    reach = fmax(reach, sqrt(q));
+                }
+            }
+            far[k] = fmin(far[k], reach);
+        }
+    }
     double e;
-    const uint32_t flags = flag_children(v, B.used, d, A.reach, e);
+    const uint32_t flags = flag_children(v, B.used, size, A.reach, e);
     const uint32_t all = (half_up(fmax(fmax(v[0], v[1]), fmax(v[2], v[3]))) + 7u) >> 3;
+    // D, and one unit more for the roundings of a walk's distance to the origin
+    double d = 0.0;
+    for (int k = 0; k < 4; ++k)
+        if (B.used[k] && !(flags >> k & 1u)) d = fmax(d, far[k]);
+    d += 1.0;
     uint4 *o = reinterpret_cast<uint4 *>(out + (L.off + j));
     o[0] = make_uint4(pl[0][0], pl[0][1], pl[0][2], pl[0][3]);
     o[1] = make_uint4(pl[1][0], pl[1][1], pl[1][2], pl[1][3]);
