@@ -487,7 +487,8 @@ enum rm_tune_key {
                                            on a batch left unsorted, 5 as 4 with a closest-hit batch of
                                            shared origins (a camera's) sorted by direction into small
                                            tiles instead (default); the four-wide walk reorders in modes
-                                           4 and 5 only large incoherent batches of large scenes */
+                                           4 and 5 only large batches: incoherent ones of large scenes,
+                                           and in mode 5 shared origins with scattered directions */
     RM_TUNE_RENDER_BLOCKS_PER_CU = 4,   /* blocks per CU of the persistent bounce kernel (default 4) */
     RM_TUNE_ADJOINT_SPLIT = 5,          /* lanes per pixel of the adjoint, each replaying a share of
                                            the pixel's samples (default 4) */

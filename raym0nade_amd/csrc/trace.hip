@@ -769,7 +769,7 @@ struct FixedWorkspace {
 // of uniform rays: 1M triangles, 300k rays 603 / 514 us, 1M 1025 / 1234, 2M
 // 1592 / 2172, 8M 4770 / 7840; 200k triangles, 1M 750 / 740, 2M 1029 / 1178; 5k
 // triangles (all in one L2), 2M 672 / 574.  Any hits among 1M triangles: 1M
-// 707 / 700, 2M 1021 / 1107.
+// 707 / 700, 2M 1021 / 1107 (all before boxes were grown, which adds 4 to 8%).
 // Mode 5's order by direction, for closest hits of one origin: a camera's rows
 // are left alone (8M rays, 1M triangles 3560 / 3023, 2M in spheres 2428 / 2440);
 // its shuffled pixels 3646 / 3973 and 2468 / 2897, with 1M rays 1019 / 1164 and

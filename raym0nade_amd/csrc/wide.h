@@ -49,11 +49,11 @@
 // loaded 511 of them (88 nodes of 64 B, 61 triangles of 48 B).  Here, before
 // boxes were grown, it loaded 287 (46 nodes, 18 runs), and 44 of a wave's 64
 // lanes took part in a node's step instead of 30.  Before and after (us,
-// launches included): 8M incoherent rays 8560 -> 4940, 8M camera rays 3440 ->
-// 2865, 100k incoherent rays among 200k triangles 583 -> 335, 1M shadow rays
-// 1013 -> 700; 1080p frame of 2M triangles at 16 spp 154 -> 114 ms.  (The growth
-// takes 3 to 5% of these batches; without the list of large triangles it took
-// 10% of scenes of small spheres on a ground.)  What bounds it now: the same data path
+// launches included): 8M incoherent rays 8550 -> 5050, 8M camera rays 3280 ->
+// 2930, 100k incoherent rays among 200k triangles 587 -> 338, 1M shadow rays
+// 1027 -> 714; 1080p frame of 2M triangles at 16 spp 106 -> 82 ms.  (The growth
+// takes 4 to 8% of these batches: 4% more nodes, 10% more instructions a node.)
+// What bounds it now: the same data path
 // (94% busy), then the vector ALUs.
 #pragma once
 #include "traverse.h"
