@@ -52,9 +52,8 @@
 // launches included): 8M incoherent rays 8550 -> 5050, 8M camera rays 3280 ->
 // 2930, 100k incoherent rays among 200k triangles 587 -> 338, 1M shadow rays
 // 1027 -> 714; 1080p frame of 2M triangles at 16 spp 106 -> 82 ms.  (The growth
-// takes 4 to 8% of these batches: 4% more nodes, 10% more instructions a node.)
-// What bounds it now: the same data path
-// (94% busy), then the vector ALUs.
+// takes 4 to 8% of these batches: up to 4% more nodes, and some 20 instructions a
+// node.)  What bounds it now: the same data path (94% busy), then the vector ALUs.
 #pragma once
 #include "traverse.h"
 
@@ -125,12 +124,11 @@ struct WideRay {
 // only, others walk the binary tree.  WIDE_SCENE bounds the growth relative to
 // |e2| over the size of a scene for |d| = 1: over 10 / 30 / 100 units, closest
 // hits among a million triangles take 0.57 / 0.73 / 1.33 of the binary walk's
-// time, 5000 take 0.65 / 0.88 / 1.75, 300 take 0.70 / 1.04 / 1.64.  WIDE_FAR bounds it for a
-// ray over its distance from the scene's middle, or half the scene's size;
-// RefWalker serves others.  Among spheres over 8 units that bound is 1.0 for
-// |d| = 20: 0.6 to 1.25 of the
-// binary walk's time; over 240 units, from outside, 3: 4 to 6 times, with
-// RefWalker 1.3.
+// time, 5000 take 0.65 / 0.88 / 1.75, 300 take 0.70 / 1.04 / 1.64.  WIDE_FAR
+// bounds it for a ray over its distance from the scene's middle, or half the
+// scene's size; RefWalker serves others.  Among spheres over 8 units that bound
+// is 1.0 for |d| = 20: 0.6 to 1.25 of the binary walk's time; over 240 units,
+// from outside, 3: 4 to 6 times, with RefWalker 1.3.
 constexpr float WIDE_ERR = 0.0126f;
 constexpr float WIDE_SCENE = 0.4f, WIDE_FAR = 1.5f;
 // The entry distances' slack below the running t_max: 3 eps_zero of rayInBox,
@@ -661,8 +659,8 @@ __device__ __forceinline__ int32_t wide_walk(const SceneView &S, V3 o, V3 d, flo
 // wave: 10k rays 223 / 241 / 258 / 278 us, 100k rays 571 / 377 / 344 / 339 us).
 // The rays of a flat scene cost the same, so a wave takes whole batches, its
 // whole share at the start where that is at most 512: claims are atomic adds
-// to one address, 12 ns each on the traces' 64-bit counter, and 64 rays a claim held 2M closest hits among
-// 36 triangles to 392 us (80 so, and 302 for 8M).
+// to one address, 12 ns each on the traces' 64-bit counter, and 64 rays a claim
+// held 2M closest hits among 36 triangles to 392 us (80 so, and 302 for 8M).
 __host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bool flat) {
     if (flat) {
         const uint32_t p = ((n - 1u) / 64u + waves) / waves * 64u;
@@ -688,8 +686,9 @@ __host__ __device__ inline uint32_t wide_per_wave(uint32_t n, uint32_t waves, bo
 // lanes then check and store their results together.  Each iteration takes
 // one kind of step: runs when at least phases / 64 of the walking lanes have
 // one, else nodes.  Every wave leaves when its rays are used up and its lanes
-// are done.  (Waves that all begin with an atomic on one address wait 6 ns
-// for each other on the renders' 32-bit counters: 50 us for a launch of 8192 with little or nothing to do.)
+// are done.  (Waves that all begin with an atomic on one address wait 6 ns for
+// each other on the renders' 32-bit counters: 50 us for a launch of 8192 with
+// little or nothing to do.)
 template <bool ANY, class Src, class Count>
 __device__ __forceinline__ void wide_loop(Src &src, Count *work, uint32_t per, float tmin, int fetch_min, int phases) {
     const uint32_t lane = threadIdx.x & 63u;

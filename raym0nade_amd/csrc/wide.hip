@@ -207,10 +207,13 @@ __device__ __forceinline__ void wide_node(const WideBuild &A, const WideLevel &L
         far[k] = sqrt(q);
         size = fmax(size, far[k]);
         if (!leaf) {
+            // (a child's D leaves its own flagged children out, which E here
+            // may count: then its box stands)
             const WideNode &C = out[ref + k];
             const double x = (double)(C.m[0] & 0xffffu) - org[0], y = (double)(C.m[0] >> 16) - org[1],
                          z = (double)(C.m[1] & 0xffffu) - org[2];
-            far[k] = fmin(far[k], sqrt(x * x + y * y + z * z) + (double)__builtin_bit_cast(_Float16, (unsigned short)(C.m[2] & 0xffffu)));
+            const double r = (double)__builtin_bit_cast(_Float16, (unsigned short)(C.m[2] & 0xffffu));
+            if (!(C.m[2] >> 28)) far[k] = fmin(far[k], sqrt(x * x + y * y + z * z) + r);
         } else {
             const uint32_t first = leaf >> LEAF_SHIFT, c = leaf & LEAF_MASK;
             double reach = 0.0;
